@@ -1,0 +1,93 @@
+"""GPU parity of the matrix-product kernel (csrc/gemm_kernel.h) at the edges
+of its tiles: rows, columns and K around the tile sizes and the 64-k chunk,
+every epilogue, both weight layouts, one and several K splits.
+
+Reference: float64 products of the same 16-bit inputs, x * gamma rounded to
+the storage type first (the operand the kernels form).  Tolerance: the fp32
+sums differ from it by less than K 2^-24 sum|x w| <= 2e-3 here, and the
+result is rounded once to 16 bits (2^-9 relative for bf16): 1e-2 covers both.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+NK, KN = 0, 1
+
+
+def _case(M, K, N, layout, dtype, gen):
+    x = torch.randn((M, K), generator=gen).to(dtype).cuda()
+    shape = (K, N) if layout == KN else (N, K)
+    ws = [(torch.randn(shape, generator=gen) * K ** -0.5).to(dtype).cuda() for _ in range(2)]
+    gamma = (1 + 0.1 * torch.randn(K, generator=gen)).to(dtype).cuda()
+    res = torch.randn((M, N), generator=gen).to(dtype).cuda()
+    return x, ws, gamma, res
+
+
+def _check(got, ref, what):
+    err = (got.double() - ref).abs()
+    bad = err > 1e-2 + 1e-2 * ref.abs()
+    print(f"[{what}] max err {err.max().item():.2e}", flush=True)
+    assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} outside 1e-2"
+
+
+@pytest.mark.parametrize("layout", [NK, KN])
+@pytest.mark.parametrize("M,K,N", [
+    (17, 8, 8),            # one chunk of 8 k, one column group
+    (31, 72, 72),          # a chunk and a piece; a tile and a piece of columns
+    (32, 1000, 520),       # whole rows of the 32-row tiles
+    (33, 1024, 200),       # one row more
+    (64, 2056, 136),       # K splits of unequal length
+    (65, 640, 1096),
+    (127, 4096, 72),       # many K splits of one column tile
+    (129, 584, 392),       # RMSNorm by its row pass from here on
+    (250, 1216, 2056),
+    (257, 64, 264),        # one row into the second 256-row tile, a single chunk
+    (600, 1088, 1544),
+])
+def test_tile_edges(M, K, N, layout):
+    import yirage_amd.fused as F
+
+    print(f"case gemm M={M} K={K} N={N} layout={layout}", flush=True)
+    gen = torch.Generator().manual_seed(M * 7 + K)
+    dtype = torch.bfloat16 if (M + K // 8) % 2 else torch.float16
+    x, (w, w3), gamma, res = _case(M, K, N, layout, dtype, gen)
+    wd, w3d = ((t if layout == KN else t.t()).double() for t in (w, w3))
+    xd = x.double()
+    for residual in (None, res):
+        out = F.linear(x, w, residual=residual, w_layout=layout)
+        _check(out, xd @ wd + (0 if residual is None else res.double()), "linear")
+        again = F.linear(x, w, residual=residual, w_layout=layout)  # tickets re-armed, same order of sums
+        assert torch.equal(out, again)
+    a = xd @ wd
+    _check(F.gated_mlp(x, w, w3, w_layout=layout), a * torch.sigmoid(a) * (xd @ w3d), "gated_mlp")
+    rs = torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    _check(F.rmsnorm_linear(x, gamma, w, w_layout=layout), ((x * gamma).double() @ wd) * rs, "rmsnorm_linear")
+    _check(F.rmsnorm_linear(x, None, w, w_layout=layout), a * rs, "rmsnorm_linear, no gamma")
+
+
+@pytest.mark.parametrize("M", [40, 300])
+def test_special_values_stay_in_their_rows(M):
+    """Inf and NaN in one row of x (and none elsewhere) reach that row only:
+    rows past M, columns past N and k past K are read as copies or zeros."""
+    import yirage_amd.fused as F
+
+    gen = torch.Generator().manual_seed(5)
+    x, (w, _), gamma, _ = _case(M, 200, 136, NK, torch.bfloat16, gen)
+    x[M - 1, 3] = float("inf")
+    x[M - 2, 199] = float("nan")
+    for out in (F.linear(x, w), F.rmsnorm_linear(x, gamma, w, w_layout=NK)):
+        assert torch.isfinite(out[: M - 2]).all()
+        assert torch.isnan(out[M - 2]).all() and not torch.isfinite(out[M - 1]).any()
+
+
+def test_more_rows_than_a_panel():
+    """More rows than one launch takes (8192), the last panel a single row."""
+    import yirage_amd.fused as F
+
+    gen = torch.Generator().manual_seed(6)
+    x, (w, _), gamma, res = _case(8193, 128, 136, NK, torch.float16, gen)
+    xd, wd = x.double(), w.t().double()
+    _check(F.linear(x, w, residual=res), xd @ wd + res.double(), "linear")
+    rs = torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    _check(F.rmsnorm_linear(x, gamma, w, w_layout=NK), ((x * gamma).double() @ wd) * rs, "rmsnorm_linear")

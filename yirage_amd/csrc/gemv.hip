@@ -1,7 +1,7 @@
 // Bandwidth-bound skinny GEMMs for gfx950 with the weight in N x K layout
 // (W[N][K], torch Linear.weight): RMSNorm+linear, gated MLP and
-// linear(+residual) for passes of up to 8 rows.  (K x N weights, and N x K
-// passes of more than 16 rows, run on the MFMA kernels of skinny.hip.)
+// linear(+residual) for passes of up to 8 rows.  (K x N weights run on the
+// MFMA kernel of skinny.hip, more than 16 rows in either layout on gemm.hip.)
 //
 // Design:
 //  * Weights stream once from HBM with 128-bit loads; every lane issues all of
@@ -17,22 +17,19 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include "gemm.h"
 #include "yr_common.h"
 
 namespace yr {
 
-// K x N weights go to the MFMA kernels of skinny.hip
+// K x N weights of up to 16 rows go to the MFMA kernel of skinny.hip
 size_t skinny_kn_workspace(int B, int K, int N, int nmat, int epi);
 int skinny_kn(const uint16_t* x, const uint16_t* gamma, const uint16_t* w0, const uint16_t* w1,
               const uint16_t* residual, uint16_t* out, int B, int K, int N, float eps, int dtype, int nmat, int epi,
-              void* ws, size_t ws_bytes, hipStream_t st, const char* name);
-// N x K weights, passes of 17..128 rows: the MFMA kernel of skinny.hip
-size_t skinny_nk128_workspace(int K, int N, int nmat, int epi);
-int skinny_nk128(const uint16_t* x, const uint16_t* gamma, const uint16_t* w0, const uint16_t* w1,
-                 const uint16_t* residual, uint16_t* out, int B, int K, int N, float eps, int dtype, int nmat,
-                 int epi, void* ws, hipStream_t st, const char* name);
+              void* ws, hipStream_t st, const char* name);
 
 enum : int { EPI_LINEAR = 0, EPI_RMSNORM = 1, EPI_GATED = 2 };
+constexpr uint32_t kOob = 0xfffffff0u;  // no buffer reaches this offset
 
 struct GemvArgs {
   const uint16_t* x;        // [B][K]
@@ -220,19 +217,16 @@ static void launch_nk(const GemvArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((gemv_nk_kernel<DT, 8, NMAT, EPI, NK_C8, NK_TROWS>), grid, dim3(NK_THREADS), 0, st, a);
 }
 
-// Rows of the pass starting with `left` rows to go: up to 128 on the MFMA
-// kernel while more than 16 remain, then chunks of up to 8 on the GEMV (each
-// pass streams the weights once).
-static int pass_rows(int left) { return left > 16 ? (left < 128 ? left : 128) : (left < 8 ? left : 8); }
+// Most rows of the weight-streaming kernels; more run on gemm.hip.
+constexpr int kFewRows = 16;
 
-static size_t nk_workspace(int B, int K, int N, int nmat, int epi) {
-  size_t need = 0;
-  for (int b0 = 0; b0 < B; b0 += pass_rows(B - b0)) {
-    const int rows = pass_rows(B - b0);
-    const size_t w = rows > 16 ? skinny_nk128_workspace(K, N, nmat, epi) : plan_gemv(rows, K, N, nmat).ws;
-    if (w > need) need = w;
+static size_t ws_for(int B, int K, int N, int layout, int nmat, int epi) {
+  if (B > kFewRows) {
+    const size_t w = gm::workspace(B, K, N, epi, layout == YR_W_NK);
+    return layout == YR_W_KN && w < kTicketBytes ? kTicketBytes : w;
   }
-  return need;
+  if (layout == YR_W_KN) return skinny_kn_workspace(B, K, N, nmat, epi);
+  return plan_gemv(B < 8 ? B : 8, K, N, nmat).ws;  // passes of up to 8 rows; the widest record
 }
 
 template <int NMAT, int EPI>
@@ -243,31 +237,33 @@ static int run_gemv(GemvArgs a, int dtype, int layout, void* ws, size_t ws_bytes
   if (dtype != YR_DTYPE_F16 && dtype != YR_DTYPE_BF16) return fail(YR_E_INVALID, "%s: dtype must be f16/bf16", name);
   if (layout != YR_W_KN && layout != YR_W_NK) return fail(YR_E_INVALID, "%s: bad weight layout", name);
   if (!a.x || !a.w0 || !a.out || (NMAT == 2 && !a.w1)) return fail(YR_E_INVALID, "%s: null pointer", name);
-  if (layout == YR_W_KN)
-    return skinny_kn(a.x, a.gamma, a.w0, a.w1, a.residual, a.out, a.B, a.K, a.N, a.eps, dtype, NMAT, EPI, ws,
-                     ws_bytes, st, name);
-  const size_t need = nk_workspace(a.B, a.K, a.N, NMAT, EPI);
+  const size_t need = ws_for(a.B, a.K, a.N, layout, NMAT, EPI);
   if (need > ws_bytes || (need && !ws))
     return fail(YR_E_WORKSPACE, "%s: workspace %zu < required %zu", name, ws_bytes, need);
-  {
-    Plan q = plan_gemv(a.B < 8 ? a.B : 8, a.K, a.N, NMAT);
-    if (q.tiles > kMaxTickets) return fail(YR_E_INVALID, "%s: N=%d too large (%d tiles)", name, a.N, q.tiles);
+  if (layout == YR_W_KN ? (a.N + 63) / 64 > kMaxTickets : (a.N + NK_TROWS - 1) / NK_TROWS > kMaxTickets)
+    return fail(YR_E_INVALID, "%s: N=%d too large", name, a.N);
+  // the product kernels reach operands by 32-bit buffer offsets
+  const size_t xrows = layout == YR_W_KN || a.B < 128 ? a.B : 128;
+  if ((layout == YR_W_KN || a.B > kFewRows) &&
+      ((size_t)a.K * a.N * 2 >= kOob || xrows * a.K * 2 >= kOob))
+    return fail(YR_E_INVALID, "%s: operands must be < 4 GiB (32-bit buffer offsets)", name);
+  if (a.B > kFewRows) {
+    const gm::Call c = {a.x, a.gamma, a.w0, a.w1, a.residual, a.out, a.B, a.K, a.N, dtype, EPI, layout == YR_W_NK,
+                        a.eps};
+    return gm::run(c, ws, st, name);
   }
+  if (layout == YR_W_KN)
+    return skinny_kn(a.x, a.gamma, a.w0, a.w1, a.residual, a.out, a.B, a.K, a.N, a.eps, dtype, NMAT, EPI, ws, st,
+                     name);
   a.ldx = a.K;
   a.ldo = a.N;
   const int B = a.B;
-  for (int b0 = 0; b0 < B; b0 += pass_rows(B - b0)) {
+  for (int b0 = 0; b0 < B; b0 += 8) {
     GemvArgs c = a;
-    c.B = pass_rows(B - b0);
+    c.B = B - b0 < 8 ? B - b0 : 8;
     c.x = a.x + (size_t)b0 * a.K;
     c.out = a.out + (size_t)b0 * a.N;
     if (a.residual) c.residual = a.residual + (size_t)b0 * a.N;
-    if (c.B > 16) {
-      const int rc = skinny_nk128(c.x, c.gamma, c.w0, c.w1, c.residual, c.out, c.B, a.K, a.N, a.eps, dtype, NMAT,
-                                  EPI, ws, st, name);
-      if (rc != YR_OK) return rc;
-      continue;
-    }
     Plan p = plan_gemv(c.B, a.K, a.N, NMAT);
     c.S = p.S;
     if (p.ws) {
@@ -287,24 +283,19 @@ using namespace yr;
 
 extern "C" {
 
-static size_t ws_for(int batch, int k, int n, int w_layout, int nmat, int epi) {
-  if (w_layout == YR_W_KN) return skinny_kn_workspace(batch, k, n, nmat, epi);
-  return nk_workspace(batch, k, n, nmat, epi);
-}
-
 size_t yr_hip_rmsnorm_linear_workspace(int batch, int k, int n, int dtype, int w_layout) {
   (void)dtype;
-  return ws_for(batch, k, n, w_layout, 1, EPI_RMSNORM);
+  return batch > 0 && k > 0 && n > 0 ? ws_for(batch, k, n, w_layout, 1, EPI_RMSNORM) : 0;
 }
 
 size_t yr_hip_gated_mlp_workspace(int batch, int k, int n, int dtype, int w_layout) {
   (void)dtype;
-  return ws_for(batch, k, n, w_layout, 2, EPI_GATED);
+  return batch > 0 && k > 0 && n > 0 ? ws_for(batch, k, n, w_layout, 2, EPI_GATED) : 0;
 }
 
 size_t yr_hip_linear_workspace(int batch, int k, int n, int dtype, int w_layout) {
   (void)dtype;
-  return ws_for(batch, k, n, w_layout, 1, EPI_LINEAR);
+  return batch > 0 && k > 0 && n > 0 ? ws_for(batch, k, n, w_layout, 1, EPI_LINEAR) : 0;
 }
 
 int yr_hip_rmsnorm_linear(const void* x, const void* gamma, const void* w, void* out, int batch, int k,
