@@ -33,6 +33,11 @@ def _check(got, ref, what):
 
 @pytest.mark.parametrize("layout", [NK, KN])
 @pytest.mark.parametrize("M,K,N", [
+    (1, 8, 8),             # the one-row kernel (N x K)
+    (1, 2056, 40),         # its second K slice; the product kernel's for the gated MLP
+    (1, 2048, 6152),       # the other side of its rule for linear and gated
+    (2, 1096, 136),        # the smallest row tile, mostly empty
+    (16, 3000, 72),        # many K splits of one column tile
     (17, 8, 8),            # one chunk of 8 k, one column group
     (31, 72, 72),          # a chunk and a piece; a tile and a piece of columns
     (32, 1000, 520),       # whole rows of the 32-row tiles
@@ -91,3 +96,16 @@ def test_more_rows_than_a_panel():
     _check(F.linear(x, w, residual=res), xd @ wd + res.double(), "linear")
     rs = torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
     _check(F.rmsnorm_linear(x, gamma, w, w_layout=NK), ((x * gamma).double() @ wd) * rs, "rmsnorm_linear")
+
+
+def test_n_by_k_weights_past_4_gib():
+    """Up to 16 rows take N x K weights of any size: every tile has its own
+    32-bit offsets.  First and last columns against the reference."""
+    import yirage_amd.fused as F
+
+    K, N = 8192, 262152
+    x = torch.randn((3, K), generator=torch.Generator().manual_seed(7)).to(torch.bfloat16).cuda()
+    w = torch.empty((N, K), dtype=torch.bfloat16, device="cuda").normal_(0.0, K ** -0.5)
+    out = F.linear(x, w)
+    for cols in (slice(0, 72), slice(N - 72, N)):
+        _check(out[:, cols], x.double() @ w[cols].double().t(), "linear")

@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const uint16_t* x, const
   float ss = 0.f;
   for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
     const uint4 v = ldg16(xr + k);
-    ss += sumsq8<DT>(v);
+    ss = sumsq8<DT>(v, ss);
     if (gamma) stg16(gr + k, scale8<DT>(v, ldg16(gamma + k)));
   }
   ss = wave_sum(ss);
@@ -56,7 +56,7 @@ constexpr int kPanelRows = 8192;   // rows per launch: bounds the row pass's cop
 // split) and the slowdown of a full chip.  Fitted to 20,000 timings (390
 // shapes of 1..2048 rows, K and N 1024..14336, every tile and split count).
 // The model only ranks: over those shapes the plan it picks is on average
-// 0.8 % (linear), 0.9 % (gated) and 0.7 % (RMSNorm in LDS) slower than the
+// 0.8 % (linear), 0.9 % (gated) and 0.6 % (RMSNorm in LDS) slower than the
 // fastest, 17 % at worst.
 struct Cost {
   float chunk[kNumCfg], chunk_full[kNumCfg], kn[kNumCfg];
@@ -70,10 +70,10 @@ constexpr Cost kCostGated = {{0.232f, 0.328f, 0.401f, 0.464f, 1.605f, 0.772f, 1.
                         {0.564f, 0.645f, 0.401f, 0.464f, 1.605f, 0.772f, 1.330f},
                         {1.640f, 1.012f, 0.973f, 1.234f, 0.827f, 1.095f, 0.992f},
                         1.67f, 6.88f, 1.25f, 0.666f, 0.147f, 0.176f};
-constexpr Cost kCostNorm = {{1.240f, 0.294f, 0.371f},
-                        {0.512f, 0.294f, 0.371f},
-                        {1.260f, 1.015f, 1.074f},
-                        5.25f, 7.88f, 0.92f, 0.819f, 0.130f, 0.250f};
+constexpr Cost kCostNorm = {{0.193f, 0.332f, 0.438f},
+                        {0.421f, 0.332f, 0.438f},
+                        {0.765f, 1.112f, 1.085f},
+                        3.12f, 7.08f, 1.25f, 1.039f, 0.067f, 0.250f};
 
 // The best plan of one kind (`pass`: RMSNorm with its row pass) and its time.
 static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* time) {
@@ -97,7 +97,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
     // 128 tile holds a fourth stage instead
     const int per_cu = lds_norm && f == C32x128 ? 1 : s.per_cu;
     const float kf = nkl ? 1.f : c.kn[f];
-    for (int sp = 1; sp <= 16; sp++) {
+    for (int sp = 1; sp <= kMaxSplits; sp++) {
       // at least 5 chunks per split (a deep pipeline has to fill), no empty
       // split, and no more workgroups than a second round of the chip holds
       if (sp > 1 && (chunks < 5 * sp || tiles * sp > 4 * kCus || tiles > kMaxTickets)) break;

@@ -53,6 +53,7 @@ struct Args {
 };
 
 constexpr int KS = 64;                   // k per chunk
+constexpr int kMaxSplits = 16;           // K splits of a tile
 constexpr uint32_t kOob = 0xfffffff0u;   // offset that is out of range for every buffer
 constexpr int kSc1 = 16;                 // buffer cache policy: sc1 (agent-scope coherence)
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -101,27 +102,29 @@ __device__ __forceinline__ uint2 lds_tr(const char* p) {
 }
 
 // x * gamma, element-wise on 8 packed values, rounded to the storage type
-// (the normalised activation the reference feeds its matmul)
+// (the normalised activation the reference feeds its matmul).  f16: the packed
+// product rounds once, as the exact fp32 product of two halves does.
 template <int DT>
 __device__ __forceinline__ uint4 scale8(uint4 x, uint4 g) {
   const uint32_t xv[4] = {x.x, x.y, x.z, x.w}, gv[4] = {g.x, g.y, g.z, g.w};
   uint32_t o[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
-    o[i] = pack2<DT>(lo16<DT>(xv[i]) * lo16<DT>(gv[i]), hi16<DT>(xv[i]) * hi16<DT>(gv[i]));
+  for (int i = 0; i < 4; i++) {
+    if constexpr (DT == DT_F16)
+      o[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, xv[i]) * __builtin_bit_cast(half2v, gv[i]));
+    else
+      o[i] = pack2<DT>(lo16<DT>(xv[i]) * lo16<DT>(gv[i]), hi16<DT>(xv[i]) * hi16<DT>(gv[i]));
+  }
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
+// s + the squares of 8 packed values, fp32
 template <int DT>
-__device__ __forceinline__ float sumsq8(uint4 x) {
-  const uint32_t xv[4] = {x.x, x.y, x.z, x.w};
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const float lo = lo16<DT>(xv[i]), hi = hi16<DT>(xv[i]);
-    s += lo * lo + hi * hi;
-  }
-  return s;
+__device__ __forceinline__ float sumsq8(uint4 x, float s) {
+  s = dot2<DT>(x.x, x.x, s);
+  s = dot2<DT>(x.y, x.y, s);
+  s = dot2<DT>(x.z, x.z, s);
+  return dot2<DT>(x.w, x.w, s);
 }
 
 // WM x WN waves; wave (wm, wn) owns rows wm BM / WM .. of the tile and
@@ -271,7 +274,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
   auto norm_wr = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-      ss[p] += sumsq8<DT>(px[p]);
+      ss[p] = sumsq8<DT>(px[p], ss[p]);
       if (a.gamma) *reinterpret_cast<uint4*>(lds + s * XB + (tid + 64 * NW * p) * 16) = scale8<DT>(px[p], pg);
     }
   };
@@ -308,22 +311,23 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
     }
   };
   // Chunk ci in stage s.  The wait lets the loads of chunks ci + 2 .. pend
-  // (RMSNorm in LDS: ci + 3 .., as chunk ci + 2 is scaled here); near the end
-  // fewer are in flight and it waits for all.  (Past the last chunk the reads
-  // find stale LDS, which no MFMA uses.)
+  // (RMSNorm in LDS: ci + 3 .., as chunk ci + 2 is read here and written back
+  // scaled before the next barrier, which is the one its first use waits for);
+  // near the end fewer are in flight and it waits for all.  (Past the last
+  // chunk the reads find stale LDS, which no MFMA uses.)
   constexpr int AHEAD = NORM ? 2 : 1;
   auto chunk = [&](int ci, auto sc, auto ldc) __attribute__((always_inline)) {
     constexpr int s = decltype(sc)::value, s1 = (s + 1) % NST, s2 = (s + 2) % NST;
     constexpr bool LD = decltype(ldc)::value;
     half(f0, f1, 1, s, std::false_type{}, 0, 0);
+    if constexpr (NORM)
+      if (ci > 0 && (LD || ci + 1 < nch)) norm_wr(s1);  // chunks 0 and 1 were scaled before the loop
     if (LD || ci + NST <= nch) wait_and_sync<(NST - 1 - AHEAD) * LPW>();
     else wait_and_sync<0>();
     if constexpr (NORM)
       if (LD || ci + 2 < nch) norm_rd(s2);
     if constexpr (!LD) issue(ci + NST, s);
     half(f1, f0, 0, s1, ldc, ci + NST, s);
-    if constexpr (NORM)
-      if (LD || ci + 2 < nch) norm_wr(s2);
   };
   auto round = [&](int ci, auto self, auto sc, auto ldc) __attribute__((always_inline)) {
     constexpr int s = decltype(sc)::value;
@@ -387,6 +391,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
     auto rec = [&](int s2, int w) __attribute__((always_inline)) {
       return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, off(s2, w), 0, kSc1));
     };
+    // every split's row sum first, in flight beside the records
+    float rs[NORM ? kMaxSplits : 1];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int s2 = 0; s2 < kMaxSplits; s2++)
+        rs[s2] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rp, tid < BM ? off(s2, NV) : kOob, 0, kSc1));
+    }
     // VG float4s of SU splits in flight (offsets past the records read zeros):
     // one split at a time, every record was a memory round trip of its own
     constexpr int VG = NV % 4 == 0 ? 4 : NV % 2 == 0 ? 2 : 1, SU = 4;
@@ -412,8 +424,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
     if constexpr (NORM) {
       if (tid < BM) {
         float sum = 0.f;
-        for (int s2 = 0; s2 < a.splits; s2++)
-          sum += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rp, off(s2, NV), 0, kSc1));
+#pragma unroll
+        for (int s2 = 0; s2 < kMaxSplits; s2++) sum += rs[s2];
         rss[tid] = sum;
       }
       __syncthreads();
