@@ -40,6 +40,7 @@ FLAGS = [
 # accumulators cost a copy in and out on every tile.
 EXTRA = {
     "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "graph_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # the product kernel's small tiles copied AGPR accumulators in and out of every chunk
     "gemm_linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_norm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

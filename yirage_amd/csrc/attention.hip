@@ -17,11 +17,10 @@
 #include <mutex>
 
 #include "yr_common.h"
+#include "attn_device.h"
 #include "attn_launch.h"
 
 namespace yr {
-
-constexpr float kLog2e = 1.4426950408889634f;
 
 // ---------------------------------------------------------------- decode
 // Streaming split-KV decode: grid = (splits, kv heads, batch) with about one
@@ -356,7 +355,6 @@ static DecPlan dec_plan(int batch, int hkv, int max_len, int page) {
 constexpr int PF_QROWS = 64;             // query rows per block (4 row waves x 16)
 constexpr int PF_KT = 64;                // kv tokens per tile
 constexpr int PF_NB = PF_KT / 16;        // 16-token MFMA blocks per tile
-constexpr float kLazy = 8.f;             // running-max slack (log2 units)
 
 struct PrefillArgs {
   const uint16_t* q;  // [B] x [Sq] rows x [Hq][D]: row r of batch b at b q_bs + r q_ld
@@ -371,25 +369,6 @@ struct PrefillArgs {
   float scale_log2;
 };
 
-// 4 consecutive 16-bit elements from LDS, transposed across each 16-lane group
-__device__ __forceinline__ uint2 lds_tr4(const uint16_t* p) {
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(const_cast<lds_v4i16*>(
-      reinterpret_cast<const lds_v4i16*>(reinterpret_cast<const __attribute__((address_space(3))) uint16_t*>(
-          reinterpret_cast<uintptr_t>(p)))));
-  return __builtin_bit_cast(uint2, r);
-}
-
-// max over lanes l and l ^ 16 (l ^ 32): a permlane swap of the value with
-// itself hands each 16-lane row its partner row, in registers (no LDS trip)
-__device__ __forceinline__ float max_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // 16-byte chunk permutation of a 256-byte LDS row: bits 1..3 = row % 8,
 // bit 0 = (row / 8) % 2.  16 consecutive rows get 16 distinct values (K
 // fragment reads, one chunk column over 16 rows), and 8 rows starting at a
@@ -401,16 +380,6 @@ __device__ __forceinline__ int pf_swz(int row) { return ((row & 7) << 1) | ((row
 // which pf_swz (even chunks for rows 0..7) does not (measured: all bank
 // conflicts of the kernel were K reads)
 __device__ __forceinline__ int pk_swz(int row) { return row & 15; }
-
-// 16 bytes per lane from global memory straight into LDS: lane l's data
-// lands at lds_base + 16 l (lds_base wave-uniform)
-__device__ __forceinline__ void lds_load16(const uint16_t* g, uint16_t* lds_base) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)(g),
-      reinterpret_cast<__attribute__((address_space(3))) void*>(
-          reinterpret_cast<__attribute__((address_space(3))) char*>(reinterpret_cast<uintptr_t>(lds_base))),
-      16, 0, 0);
-}
 
 // HPW heads per wave, HG head groups (of 4 row waves) per workgroup
 template <int DT, int HPW, int HG>

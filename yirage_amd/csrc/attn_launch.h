@@ -26,4 +26,15 @@ int prefill_launch(const char* nm, const void* q, const void* k, const void* v, 
                    int hq, int hkv, int d, int causal, int dtype, long long q_bs, int q_ld, long long kv_bs, int kv_ld,
                    long long o_bs, int o_ld, float scale, hipStream_t st);
 
+// Attention of a kernel graph on its operands as they lie: Q / V / O rows and
+// K's head-dim rows contiguous (strides of group, row, element; multiples of 8
+// but the last).  _direct says whether the kernel takes the shape, _launch also
+// needs 16-byte aligned operands and the zeroed tickets + records of _workspace.
+bool graph_attn_direct(int G, int M, int L, int d, const long long* sq, const long long* sk, const long long* sv,
+                       const long long* so);
+size_t graph_attn_direct_workspace(int G, int M, int L, int d);
+int graph_attn_launch(const char* nm, const void* q, const void* k, const void* v, void* out, int G, int M, int L,
+                      int d, const long long* sq, const long long* sk, const long long* sv, const long long* so,
+                      float scale, int dtype, void* workspace, hipStream_t st);
+
 }  // namespace yr

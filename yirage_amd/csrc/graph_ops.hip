@@ -494,7 +494,8 @@ __global__ void page_iota_kernel(int32_t* indptr, int32_t* indices, int32_t* len
 // ------------------------------------------------------------------ graph attention
 // O[g] = softmax(scale * Q[g] K[g]) V[g] with Q [G][M][d], K [G][d][L]
 // (the kernel-graph operand: its rows are head dims), V [G][L][d], each given
-// by three element strides.  Up to 16 query rows per group (a power of two)
+// by three element strides.  Where the operands can be read as they lie, the
+// kernel of graph_attn.hip takes them; else up to 16 query rows per group (a power of two)
 // run on the split-KV decode kernel over an identity page table (one page of
 // L tokens per group), more on the flash-attention prefill kernel.  Operands
 // not already laid out as [G][rows][128] contiguous are packed into the
@@ -594,7 +595,11 @@ extern "C" {
 size_t yr_hip_graph_attention_workspace(int G, int M, int L, int d, const int64_t* strides12) {
   if (G <= 0 || M <= 0 || L <= 0 || d <= 0 || d > 128 || !strides12) return 0;
   const long long* s = reinterpret_cast<const long long*>(strides12);
-  return attn_plan(G, M, L, d, s, s + 3, s + 6, s + 9).total;
+  const size_t packed = attn_plan(G, M, L, d, s, s + 3, s + 6, s + 9).total;
+  if (!graph_attn_direct(G, M, L, d, s, s + 3, s + 6, s + 9)) return packed;
+  // both: a call whose operands are not 16-byte aligned still packs them
+  const size_t direct = graph_attn_direct_workspace(G, M, L, d);
+  return direct > packed ? direct : packed;
 }
 
 int yr_hip_graph_attention(const void* q, const void* k, const void* v, void* out, int G, int M, int L, int d,
@@ -607,6 +612,15 @@ int yr_hip_graph_attention(const void* q, const void* k, const void* v, void* ou
   if (dtype != YR_DTYPE_F16 && dtype != YR_DTYPE_BF16) return fail(YR_E_INVALID, "%s: dtype", nm);
   const long long* s = reinterpret_cast<const long long*>(strides12);
   const long long *sq = s, *sk = s + 3, *sv = s + 6, *so = s + 9;
+  const bool direct = graph_attn_direct(G, M, L, d, sq, sk, sv, so) &&
+                      (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) == 0;
+  if (direct) {
+    const size_t need = yr_hip_graph_attention_workspace(G, M, L, d, strides12);
+    if (need > workspace_bytes || !workspace)
+      return fail(YR_E_WORKSPACE, "%s: workspace %zu < %zu", nm, workspace_bytes, need);
+    return graph_attn_launch(nm, q, k, v, out, G, M, L, d, sq, sk, sv, so, scale, dtype, workspace,
+                             (hipStream_t)stream);
+  }
   const AttnPlan p = attn_plan(G, M, L, d, sq, sk, sv, so);
   if (p.total > workspace_bytes || (p.total && !workspace))
     return fail(YR_E_WORKSPACE, "%s: workspace %zu < %zu", nm, workspace_bytes, p.total);
