@@ -4,17 +4,17 @@
 //   grid = (kv splits, kv heads, batch), about one workgroup per CU; one
 //   workgroup = 8 waves covers a chunk of tokens of one (sequence, kv head)
 //   for all G = Hq/Hkv query heads of the group.  Q.K^T runs on MFMA 16x16x32
-//   with the K rows as the B operand straight from HBM (16-byte loads, no
-//   LDS); P.V runs on MFMA too, V going through LDS and coming back as B
-//   fragments by transposing reads.  Every wave streams its own 32-token
-//   blocks with an online softmax; the 8 waves merge in LDS, and
-//   splits merge through the workspace with the last-arriving workgroup
+//   with the K rows as the B operand, P.V too, with V as B fragments by
+//   transposing reads; both come from HBM straight into LDS.  Every wave
+//   streams its own 32-token blocks with an online softmax; the 8 waves merge
+//   in LDS, and splits merge through the workspace with the last-arriving workgroup
 //   (atomic ticket) writing the output.
 //
 // Prefill (MFMA-bound): flash attention, one workgroup per (64 query rows,
 //   q head, batch); K tiles and transposed V tiles are staged in LDS, S = Q K^T
 //   and O += P V both on MFMA 16x16x32, fp32 running max/sum per row.
 #include <mutex>
+#include <type_traits>
 
 #include "yr_common.h"
 #include "attn_device.h"
@@ -26,8 +26,8 @@ namespace yr {
 // Streaming split-KV decode: grid = (splits, kv heads, batch) with about one
 // workgroup per CU in total; a workgroup (8 waves) owns `chunk` tokens of one
 // (sequence, kv head).  Its page ids are staged in LDS first, so no K/V load
-// waits on a page-table load.  The waves stream 32-token blocks (K straight
-// from HBM as MFMA B fragments, V through LDS), keep an online softmax per
+// waits on a page-table load.  The waves stream 32-token blocks through their
+// own LDS slots, keep an online softmax per
 // head row, and the 8 waves then the splits merge
 // (splits through fp32 records, the last workgroup to arrive writing out).
 constexpr int DEC_WAVES = 8;
@@ -62,22 +62,34 @@ __device__ uint64_t g_dec_prof[4096 * 8];
 // lies in one page, whose id each wave reads with one scalar load when it
 // issues the block (no page-table staging before the first K/V load);
 // otherwise the split's page ids are staged in LDS first.
-template <int DT, int G, bool PG32>
+// DMA: K and V go straight to LDS (16-byte aligned caches; others pass through
+// registers).
+// Bound by HBM and by how much of it the waves keep in flight.  Direct loads of
+// whole 256-byte token rows, K and V of a wave in turn, take 25.4 us for 8
+// ragged sequences of 2..4 K tokens (8 kv heads, 105 MB) and 30.1 us for 8 of 4
+// K tokens (134 MB, 4.5 TB/s); loads into registers, where K touched 64 bytes of
+// a row per instruction, took 27.1 and 32.0.  More than one workgroup per CU is
+// slower (8 ragged sequences in 512 workgroups: 32.9 us with register loads).
+template <int DT, int G, bool PG32, bool DMA>
 __global__ __launch_bounds__(DEC_THREADS) void gqa_decode_kernel(DecodeArgs a) {
   constexpr int D = 128;
   const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // uniform
   const int len = a.kv_len[b];
   const int c0 = split * a.chunk, c1 = min(len, c0 + a.chunk);
   const size_t tok_stride = (size_t)a.Hkv * D;  // elements between tokens in a page
   DPROF(0)
 
-  constexpr int LDV = D + 8;       // padded V rows: transposing reads without bank conflicts
   constexpr int LDP = DEC_BLK + 8;
-  static_assert(G * D * 4 <= DEC_BLK * LDV * 2, "wave's O must fit its V slot");
-  __shared__ int s_pg[DEC_MAXPG];
-  // per wave: the V block (then, after the loop, the wave's O as fp32 [G][D])
-  __shared__ __attribute__((aligned(16))) uint16_t s_v[DEC_WAVES][DEC_BLK * LDV];
+  static_assert(G * D * 4 <= DEC_BLK * D * 2, "wave's O must fit its V slot");
+  __shared__ int s_pg[PG32 ? 1 : DEC_MAXPG];
+  // per wave: its K block and its V block (then, after the loop, the wave's O
+  // as fp32 [G][D]): 256-byte token rows whose 16-byte chunks are permuted by
+  // row, K's by row % 16 (16-byte reads of 16 rows), V's in pairs by v_swz
+  // (transposing reads of 8 rows, 32 bytes each, per two 16-lane groups)
+  __shared__ __attribute__((aligned(16))) uint16_t s_k[DEC_WAVES][DEC_BLK * D];
+  __shared__ __attribute__((aligned(16))) uint16_t s_v[DEC_WAVES][DEC_BLK * D];
   __shared__ __attribute__((aligned(16))) uint16_t s_p[DEC_WAVES][16 * LDP];  // P as 16-bit [row][token]
   __shared__ float s_m[DEC_WAVES][G], s_l[DEC_WAVES][G];
 
@@ -108,39 +120,29 @@ __global__ __launch_bounds__(DEC_THREADS) void gqa_decode_kernel(DecodeArgs a) {
     const int pg = s_pg[t / a.page - pg0];
     return ((size_t)pg * a.page + t % a.page) * tok_stride + (size_t)hk * D;
   };
-  struct Blk {
-    uint4 k[2][4];  // [16-token tile j][k step s]: token 16 j + lane % 16, d = 32 s + 8 (lane / 16)
-    uint4 v[8];     // token lane / 16 + 4 i, d = 8 (lane % 16)
-  };
   // the page table through the scalar path (read-only for the launch)
   const __attribute__((address_space(4))) int32_t* kvi =
       reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(a.kv_indices));
-  auto issue = [&](Blk& bk, int blk) __attribute__((always_inline)) {
+  // direct global -> LDS loads, 4 whole token rows each: lane l fills physical
+  // chunk l % 16 of row 4 u + l / 16
+  auto v_swz = [](int row) __attribute__((always_inline)) { return (row & 3) | (((row >> 3) & 1) << 2); };
+  auto issue = [&](int blk, auto is_k_c) __attribute__((always_inline)) {
+    constexpr bool IS_K = decltype(is_k_c)::value;
     const int tb = __builtin_amdgcn_readfirstlane(c0 + blk * DEC_BLK);
-    if constexpr (PG32) {
-      // tokens tb .. tb + 31 (clamped to c1 - 1, the same block) share a page
-      const int pg = kvi[pbase + tb / a.page];
-      auto off32 = [&](int t) __attribute__((always_inline)) -> size_t {
-        t = min(t, c1 - 1);
-        return ((size_t)pg * a.page + t % a.page) * tok_stride + (size_t)hk * D;
-      };
+    const uint16_t* cache = IS_K ? a.kc : a.vc;
+    // PG32: tokens tb .. tb + 31 (clamped to c1 - 1, the same block) share a page
+    if constexpr (PG32) cache += ((size_t)kvi[pbase + tb / a.page] * a.page + tb % a.page) * tok_stride + (size_t)hk * D;
 #pragma unroll
-      for (int n = 0; n < 2; n++) {
-        const size_t off = off32(tb + 16 * n + lane % 16) + (lane / 16) * 8;
-#pragma unroll
-        for (int s = 0; s < 4; s++) bk.k[n][s] = ldg16(a.kc + off + 32 * s);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; i++) bk.v[i] = ldg16(a.vc + off32(tb + lane / 16 + 4 * i) + (lane % 16) * 8);
-    } else {
-#pragma unroll
-      for (int n = 0; n < 2; n++) {
-        const size_t off = tok_off(tb + 16 * n + lane % 16) + (lane / 16) * 8;
-#pragma unroll
-        for (int s = 0; s < 4; s++) bk.k[n][s] = ldg16(a.kc + off + 32 * s);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; i++) bk.v[i] = ldg16(a.vc + tok_off(tb + lane / 16 + 4 * i) + (lane % 16) * 8);
+    for (int u = 0; u < DEC_BLK / 4; u++) {
+      const int row = 4 * u + lane / 16, chunk = 8 * ((lane % 16) ^ (IS_K ? row & 15 : 2 * v_swz(row)));
+      const uint16_t* src;
+      if constexpr (PG32)
+        src = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(cache) +
+                                                2u * (uint32_t)(min(row, c1 - 1 - tb) * (int)tok_stride + chunk));
+      else src = cache + tok_off(tb + row) + chunk;
+      uint16_t* dst = (IS_K ? s_k[wave] : s_v[wave]) + 4 * u * D;
+      if constexpr (DMA) lds_load16(src, dst);
+      else *reinterpret_cast<uint4*>(dst + 8 * lane) = ldg16(src);
     }
   };
 
@@ -152,26 +154,41 @@ __global__ __launch_bounds__(DEC_THREADS) void gqa_decode_kernel(DecodeArgs a) {
   f32x4 o[D / 16];
 #pragma unroll
   for (int n = 0; n < D / 16; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint16_t* ks = s_k[wave];
   uint16_t* vs = s_v[wave];
   uint16_t* ps = s_p[wave];
+  uint32_t koff[4];  // K fragment of step s: token lane % 16 (+ 16 n), d 32 s + 8 (lane / 16) ..
+#pragma unroll
+  for (int i = 0; i < 4; i++) koff[i] = (lane % 16) * D + 8 * ((4 * i + lane / 16) ^ (lane % 16));
+  uint32_t voff[D / 16];  // V fragment of dims 16 n: tokens 8 (lane / 16) + e (and + 4)
+  {
+    const int row = 8 * (lane / 16) + (lane % 16) / 4;
+#pragma unroll
+    for (int n = 0; n < D / 16; n++) voff[n] = row * D + 16 * (n ^ v_swz(row)) + 4 * (lane % 4);
+  }
 
   // S = Q K^T and P V both on MFMA 16x16x32.  P goes through LDS as 16-bit
   // values (the A operand wants 8 consecutive tokens per lane), V through LDS
   // unchanged and comes back as B fragments by transposing reads.  Rows past G
   // hold finite values from zero Q rows and are never written out.
-  auto consume = [&](const Blk& bk, int blk) __attribute__((always_inline)) {
-    const int tb = c0 + blk * DEC_BLK;
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      *reinterpret_cast<uint4*>(vs + (lane / 16 + 4 * i) * LDV + (lane % 16) * 8) = bk.v[i];
+  // The wave's next K block is requested as soon as this one's fragments are
+  // read, its next V block after P V, so one of the two is always in flight.
+  // LAST: there is no next block (a copy of its own: every path then knows how
+  // many loads are in flight).
+  auto consume = [&](int blk, auto last_c) __attribute__((always_inline)) {
+    constexpr bool LAST = decltype(last_c)::value;
+    const int tb = c0 + blk * DEC_BLK, nxt = blk + DEC_WAVES;
     f32x4 sc[2];
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // K has landed, V (8 loads) may be on its way
 #pragma unroll
     for (int n = 0; n < 2; n++) {
       f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < 4; s++) c = mfma16<DT>(qf[s], bk.k[n][s], c);
+      for (int s = 0; s < 4; s++) c = mfma16<DT>(qf[s], *reinterpret_cast<const uint4*>(&ks[koff[s] + 16 * n * D]), c);
       sc[n] = c;
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every K fragment is in registers
+    if constexpr (!LAST) issue(nxt, std::true_type{});
     float alpha[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -202,34 +219,28 @@ __global__ __launch_bounds__(DEC_THREADS) void gqa_decode_kernel(DecodeArgs a) {
     // LDS operations of one wave complete in order; the asm keeps the
     // compiler from moving the reads above the writes.
     asm volatile("" ::: "memory");
+    if constexpr (!LAST) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // V; the next K is on its way
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const uint4 pa = *reinterpret_cast<const uint4*>(ps + (lane % 16) * LDP + (lane / 16) * 8);
 #pragma unroll
     for (int n = 0; n < D / 16; n++) {
 #pragma unroll
       for (int i = 0; i < 4; i++) o[n][i] *= alpha[i];
-      o[n] = mfma16<DT>(pa, b_frag(vs + 16 * n, LDV, 0, lane), o[n]);
+      const uint2 lo = lds_tr4(&vs[voff[n]]), hi = lds_tr4(&vs[voff[n] + 4 * D]);
+      o[n] = mfma16<DT>(pa, make_uint4(lo.x, lo.y, hi.x, hi.y), o[n]);
     }
-    asm volatile("" ::: "memory");  // the next block's writes stay after these reads
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every V and P fragment is in registers
+    if constexpr (!LAST) issue(nxt, std::false_type{});
   };
 
   // Wave w takes blocks w, w + 8, ... (a fixed order, so results do not
-  // depend on timing).  One block in flight per wave: with every workgroup
-  // resident that is ~64 MiB queued at once, and deeper queues only lengthen
-  // the tail.
-  int cur = wave;
-  if (cur < nblk) {
-    Blk bk;
-    issue(bk, cur);
-    bool first = true;
-    for (;;) {
-      const int nxt = cur + DEC_WAVES;
-      consume(bk, cur);
-      if (first) DPROF(2)
-      first = false;
-      if (nxt >= nblk) break;
-      issue(bk, nxt);
-      cur = nxt;
-    }
+  // depend on timing).
+  if (wave < nblk) {
+    issue(wave, std::true_type{});
+    issue(wave, std::false_type{});
+    int blk = wave;
+    for (; blk + DEC_WAVES < nblk; blk += DEC_WAVES) consume(blk, std::false_type{});
+    consume(blk, std::true_type{});
   }
 
   DPROF(3)
@@ -277,43 +288,72 @@ __global__ __launch_bounds__(DEC_THREADS) void gqa_decode_kernel(DecodeArgs a) {
   DPROF(4)
   if (a.splits == 1) return;
 
-  // ---- split merge by the last workgroup of this (b, hk): every record in
-  // flight at once (one thread per (g, d, split lane j of P))
+  // ---- split merge by the last workgroup of this (b, hk).  A thread takes 4
+  // dims of one head over every SG-th split, 8 records in flight, and the SG
+  // partial results meet in LDS (a fixed order).  Bound by the records' trip
+  // past the L2: one or two trips instead of one per 16 splits with 4-byte
+  // loads (2 sequences x 2 kv heads, 64 splits each: 23.1 -> 17.8 us a call).
   if (!arrive_last(&a.tickets[b * a.Hkv + hk], a.splits)) return;
   DPROF(5)
-  for (int idx = tid; idx < G * D; idx += DEC_THREADS) {
-    const int g = idx / D, d = idx % D;
-    float M = -INFINITY, L = 0.f, O = 0.f;
-    for (int s0 = 0; s0 < a.splits; s0 += 16) {
-      float mv[16], lv[16], ov[16];
+  constexpr int ITEMS = G * D / 4, SG = DEC_THREADS / ITEMS, MU = 8;
+  static_assert(ITEMS * SG == DEC_THREADS && DEC_THREADS * 16 <= (int)sizeof(s_v), "one item per thread");
+  float4* so = reinterpret_cast<float4*>(&s_v[0][0]);
+  __shared__ float2 s_sg[SG][G];
+  {
+    const int item = tid % ITEMS, j = tid / ITEMS, g = item / (D / 4), d0 = item % (D / 4) * 4;
+    float M = -INFINITY, L = 0.f;
+    float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = j; s0 < a.splits; s0 += SG * MU) {
+      float mv[MU], lv[MU];
+      float4 ov[MU];
 #pragma unroll
-      for (int u = 0; u < 16; u++) {
-        if (s0 + u < a.splits) {
-          const float* rec = rec_base + ((size_t)(s0 + u) * G + g) * REC;
+      for (int u = 0; u < MU; u++) {
+        mv[u] = -INFINITY;
+        lv[u] = 0.f;
+        ov[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (s0 + u * SG < a.splits) {
+          const float* rec = rec_base + ((size_t)(s0 + u * SG) * G + g) * REC;
           mv[u] = ld_agent(rec + D);
           lv[u] = ld_agent(rec + D + 1);
-          ov[u] = ld_agent(rec + d);
-        } else {
-          mv[u] = -INFINITY;
-          lv[u] = 0.f;
-          ov[u] = 0.f;
+          ov[u] = ld_agent4(rec + d0);
         }
       }
       float mb = M;
 #pragma unroll
-      for (int u = 0; u < 16; u++) mb = fmaxf(mb, mv[u]);
+      for (int u = 0; u < MU; u++) mb = fmaxf(mb, mv[u]);
       const float f0 = M == -INFINITY ? 0.f : exp2f(M - mb);
       L *= f0;
-      O *= f0;
+      O.x *= f0; O.y *= f0; O.z *= f0; O.w *= f0;
 #pragma unroll
-      for (int u = 0; u < 16; u++) {
+      for (int u = 0; u < MU; u++) {
         const float f = mv[u] == -INFINITY ? 0.f : exp2f(mv[u] - mb);
         L += lv[u] * f;
-        O += ov[u] * f;
+        O.x += ov[u].x * f; O.y += ov[u].y * f; O.z += ov[u].z * f; O.w += ov[u].w * f;
       }
       M = mb;
     }
-    a.out[((size_t)b * a.Hq + (size_t)hk * G + g) * D + d] = (uint16_t)st_elem<DT>(L > 0.f ? O / L : 0.f);
+    if constexpr (SG > 1) {
+      so[tid] = O;
+      if (d0 == 0) s_sg[j][g] = make_float2(M, L);
+      __syncthreads();
+      if (j > 0) return;
+      float mb = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < SG; u++) mb = fmaxf(mb, s_sg[u][g].x);
+      L = 0.f;
+      O = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int u = 0; u < SG; u++) {
+        const float2 ml = s_sg[u][g];
+        const float4 v = so[u * ITEMS + item];
+        const float f = ml.x == -INFINITY ? 0.f : exp2f(ml.x - mb);
+        L += ml.y * f;
+        O.x += v.x * f; O.y += v.y * f; O.z += v.z * f; O.w += v.w * f;
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    *reinterpret_cast<uint2*>(a.out + ((size_t)b * a.Hq + (size_t)hk * G + g) * D + d0) =
+        make_uint2(pack2<DT>(O.x * inv, O.y * inv), pack2<DT>(O.z * inv, O.w * inv));
   }
   DPROF(6)
 }
@@ -803,18 +843,24 @@ int yr::gqa_decode_launch(const char* nm, const void* q, const void* k_cache, co
   if (!(scale > 0.f)) return fail(YR_E_INVALID, "%s: scale must be positive", nm);
   a.scale_log2 = kLog2e * scale;
   dim3 grid(a.splits, hkv, batch);
+  // direct loads into LDS need aligned rows (they are 256 bytes apart)
+  const bool dma = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
+#define YR_DEC_DT(G_, PG_, DMA_)                                                                          \
+  {                                                                                                       \
+    if (dtype == YR_DTYPE_F16)                                                                            \
+      hipLaunchKernelGGL((gqa_decode_kernel<DT_F16, G_, PG_, DMA_>), grid, dim3(DEC_THREADS), 0, st, a);   \
+    else                                                                                                  \
+      hipLaunchKernelGGL((gqa_decode_kernel<DT_BF16, G_, PG_, DMA_>), grid, dim3(DEC_THREADS), 0, st, a);  \
+  }
 #define YR_DEC(G_)                                                                                        \
   if (G == G_) {                                                                                          \
-    if (page_size % DEC_BLK == 0) {                                                                       \
-      if (dtype == YR_DTYPE_F16) hipLaunchKernelGGL((gqa_decode_kernel<DT_F16, G_, true>), grid, dim3(DEC_THREADS), 0, st, a); \
-      else hipLaunchKernelGGL((gqa_decode_kernel<DT_BF16, G_, true>), grid, dim3(DEC_THREADS), 0, st, a);   \
-    } else {                                                                                              \
-      if (dtype == YR_DTYPE_F16) hipLaunchKernelGGL((gqa_decode_kernel<DT_F16, G_, false>), grid, dim3(DEC_THREADS), 0, st, a); \
-      else hipLaunchKernelGGL((gqa_decode_kernel<DT_BF16, G_, false>), grid, dim3(DEC_THREADS), 0, st, a);  \
-    }                                                                                                     \
+    if (!dma) YR_DEC_DT(G_, false, false)                                                                 \
+    else if (page_size % DEC_BLK == 0) YR_DEC_DT(G_, true, true)                                          \
+    else YR_DEC_DT(G_, false, true)                                                                       \
   }
   YR_DEC(1) YR_DEC(2) YR_DEC(4) YR_DEC(8) YR_DEC(16)
 #undef YR_DEC
+#undef YR_DEC_DT
   YR_CHECK_LAUNCH(nm);
   return YR_OK;
 }

@@ -37,7 +37,7 @@ struct Args {
 
 // Bound by LDS reads and the softmax between them where many rows share a
 // tile, by the split merge for few.  16 groups of 256 rows, 4096 tokens, d =
-// 64, f16: 19.5 us (4.3 GFLOP), against 126 us for packing Q, K, V to d = 128
+// 64, f16: 17.6 us (4.3 GFLOP), against 126 us for packing Q, K, V to d = 128
 // and the prefill kernel on 64 workgroups.
 template <int DT, int D, int RW, int KW, int RB>
 __global__ __launch_bounds__(64 * RW * KW, 2) void graph_attn_kernel(Args a) {
@@ -331,7 +331,7 @@ struct Plan {
 // fastest tile while the tokens have to be split to fill the chip: the last
 // workgroup merges all splits of its rows, so small tiles merge in parallel
 // (16 groups of 256 rows over 4096 tokens, d = 64: 19.5 us, 22.4 with 64 rows,
-// 28.5 with 128, 28.8 with 16).  Without splits a fragment read should feed
+// 28.5 with 128, 28.8 with 16, all before the reads' waits were loosened).  Without splits a fragment read should feed
 // more rows: 64 (8 groups of 4096 rows, 2048 tokens, d = 128: 56 us, 72 with
 // 32 rows), or 128 at d = 64 (16 groups: 53 us, 66 with 64 rows); at d = 128
 // 128 rows spill registers.  Two workgroups per CU and at least 256 tokens per
