@@ -68,12 +68,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_
 // for these loads (it cannot tell which LDS stage one writes and would wait
 // for all of them before any LDS read); the kernel orders them itself
 // (s_waitcnt vmcnt and a barrier before a stage is read, a barrier after the
-// last read of a stage before it is refilled).
+// last read of a stage before it is refilled).  The s_nop is the wait state
+// that a load reading M0 needs after a scalar write of it: the compiler
+// inserts none inside inline assembly.
 __device__ __forceinline__ void bload_lds16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds"
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds"
                :
                : "v"(off), "s"(__builtin_amdgcn_readfirstlane(lds)), "s"(r), "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory");
+               : "memory", "m0");
 }
 
 // At most N of this wave's vector-memory operations and none of its LDS

@@ -807,11 +807,13 @@ constexpr int XS_QUARTER = XS_ELEMS / 4;  // QUAD staging buffers
 // lds_block + 16 l, lds_block wave-uniform), agent-coherent (sc1); an offset
 // past the buffer writes zeros.  Inline assembly, so the compiler inserts no
 // waits of its own for these loads: the sync wave orders them itself
-// (s_waitcnt vmcnt, then the barrier that publishes the block).
+// (s_waitcnt vmcnt, then the barrier that publishes the block).  The s_nop is
+// the wait state between a scalar write of M0 and a load that reads it, which
+// the compiler does not insert inside inline assembly.
 __device__ __forceinline__ void bload_lds16_sc1(__amdgpu_buffer_rsrc_t r, uint32_t off, void* lds_block) {
   const uint32_t lds = __builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds_block));
-  asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, 0 offen sc1 lds"
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, 0 offen sc1 lds"
                :
                : "v"(off), "s"(lds), "s"(r)
                : "memory", "m0");
