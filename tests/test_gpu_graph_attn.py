@@ -108,3 +108,25 @@ def test_infinite_scores_and_weights():
     assert _call(q, k, v, out, 0.125)[0] == 0
     assert (out[:, 0] == 0).all()
     _check(out[:, 1:], q[:, 1:], k, v, 0.125)
+
+
+@pytest.mark.parametrize("M", [1, 3, 33])
+def test_long_tail_of_small_weights(M):
+    """Weights that round to 0 in f16 beside the row's maximum (2^-26 each)
+    still count in the row sum, which is fp32: a token of weight 1 and V = 1,
+    then 65535 whose V is +1 and -1 in turn, give 1 / (1 + 65535 2^-26).  The
+    numerator loses at most one such weight (2^-26), the sum is fp32, and the
+    result is rounded once to f16."""
+    G, L, d, dt = 512, 65536, 64, torch.float16
+    print("case tail", M, flush=True)
+    q = torch.zeros((G, M, d), dtype=dt, device="cuda")
+    q[..., 0] = 1
+    k = torch.zeros((1, d, L), dtype=dt, device="cuda")
+    k[:, 0] = -26
+    k[:, 0, 0] = 0
+    v = torch.ones((1, L, d), dtype=dt, device="cuda")
+    v[:, 2::2] = -1
+    out = torch.empty_like(q)
+    assert _call(q, k.expand(G, d, L), v.expand(G, L, d), out, math.log(2))[0] == 0
+    ref = 1 / (1 + 65535 * 2.0 ** -26)
+    assert (out.double() - ref).abs().max().item() <= 2.0 ** -12 + 2.0 ** -20

@@ -124,17 +124,15 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void graph_attn_kernel(Args a) {
     for (int s = 0; s < NS; s++)
       qf[rb][s] = ldg16(a.q + g * a.q_bs + min(qr0 + 16 * rb, a.M - 1) * a.q_ld + 32 * s + 8 * grp);
 
-  f32x4 acc[RB][NDT], lsum[RB];  // O^T: row d 16 dt + 4 grp + i, column query row
-  float m_i[RB];
+  f32x4 acc[RB][NDT];  // O^T: row d 16 dt + 4 grp + i, column query row
+  float m_i[RB], l_i[RB];  // l: this lane's tokens only until the loop ends
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) {
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++) acc[rb][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    lsum[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    l_i[rb] = 0.f;
     m_i[rb] = -INFINITY;
   }
-  const uint32_t one2 = st_elem<DT>(1.f) * 0x10001u;
-  const uint4 ones = make_uint4(one2, one2, one2, one2);
 
   auto step = [&](int t, const uint16_t* st, auto edge_c) __attribute__((always_inline)) {
     constexpr bool EDGE = decltype(edge_c)::value;
@@ -176,25 +174,28 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void graph_attn_kernel(Args a) {
         const float mnew = grow ? mx : m_i[rb];
         const float alpha = m_i[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i[rb] - mnew);
         m_i[rb] = mnew;
-        lsum[rb] *= alpha;
+        l_i[rb] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) acc[rb][dt] *= alpha;
       }
       const float mref = m_i[rb] == -INFINITY ? 0.f : m_i[rb];
-      float p[NB][4];
+      // the row sum takes P before it is rounded for P V: an f16 P far below
+      // the row's maximum rounds to 0, and many such tokens have a weight
+      float p[NB][4], ls = 0.f;
 #pragma unroll
       for (int n = 0; n < NB; n++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) p[n][i] = __builtin_amdgcn_exp2f(fmaf(sc[rb][n][i], a.scale_log2, -mref));
-      // k slot 8 grp + 4 j + i of step m <-> token 32 m + 16 j + 4 grp + i;
-      // the row sum of the rounded P is one more MFMA, with a row of ones
+        for (int i = 0; i < 4; i++) {
+          p[n][i] = __builtin_amdgcn_exp2f(fmaf(sc[rb][n][i], a.scale_log2, -mref));
+          ls += p[n][i];
+        }
+      l_i[rb] += ls;
+      // k slot 8 grp + 4 j + i of step m <-> token 32 m + 16 j + 4 grp + i
 #pragma unroll
-      for (int m = 0; m < NB / 2; m++) {
+      for (int m = 0; m < NB / 2; m++)
         pb[rb][m] = make_uint4(pack2<DT>(p[2 * m][0], p[2 * m][1]), pack2<DT>(p[2 * m][2], p[2 * m][3]),
                                pack2<DT>(p[2 * m + 1][0], p[2 * m + 1][1]),
                                pack2<DT>(p[2 * m + 1][2], p[2 * m + 1][3]));
-        lsum[rb] = mfma16<DT>(ones, pb[rb][m], lsum[rb]);
-      }
     }
 #pragma unroll
     for (int m = 0; m < NB / 2; m++)
@@ -218,9 +219,8 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void graph_attn_kernel(Args a) {
     if (t + 1 < ntile) tile(t + 1, st1, st0);
   }
 
-  float l_i[RB];
 #pragma unroll
-  for (int rb = 0; rb < RB; rb++) l_i[rb] = lsum[rb][0];
+  for (int rb = 0; rb < RB; rb++) l_i[rb] = add_xor32(add_xor16(l_i[rb]));
   auto weight = [](float m, float M) __attribute__((always_inline)) {
     return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
   };
