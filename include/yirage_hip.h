@@ -289,6 +289,19 @@ int yr_hip_run_fused(int op_kind, int n_in, const void* const* inputs, int n_out
  * workspace layout is shared by every kind (tickets first), so one
  * zero-filled buffer of the maximum over a graph's steps serves them all. */
 size_t yr_hip_fused_workspace(int op_kind, int n_params, const int64_t* params);
+/* The kernel an op runs on (host only; `aligned`: every operand 16-byte
+ * aligned).  plan6[0]: YR_PLAN_ONE_ROW, plan6[1..3] = {1, columns, K slices};
+ * YR_PLAN_PRODUCT, {tile rows, tile columns (of all matrices), K splits}, and
+ * plan6[4] = RMSNorm by a row pass, plan6[5] = operands through registers;
+ * YR_PLAN_ATTENTION (graph attention on the operands as they lie), {query
+ * rows, tokens per split, splits}; YR_PLAN_PACKED (graph attention on the
+ * decode or prefill kernel).  YR_E_INVALID for other kinds and shapes that are
+ * refused. */
+#define YR_PLAN_ONE_ROW 0
+#define YR_PLAN_PRODUCT 1
+#define YR_PLAN_ATTENTION 2
+#define YR_PLAN_PACKED 3
+int yr_hip_fused_plan(int op_kind, int n_params, const int64_t* params, int aligned, int* plan6);
 
 /* ------------------------------------------------------- persistent kernel */
 /* Task graph of the persistent megakernel, built on the host (no GPU needed).

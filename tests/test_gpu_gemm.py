@@ -71,6 +71,48 @@ def test_tile_edges(M, K, N, layout):
     _check(F.rmsnorm_linear(x, None, w, w_layout=layout), a * rs, "rmsnorm_linear, no gamma")
 
 
+def _odd(t):
+    """The same values one element off a 16-byte boundary."""
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("layout", [NK, KN])
+@pytest.mark.parametrize("M,K,N", [
+    (1, 4096, 4096),       # product kernel: one row, K splits
+    (3, 8, 8),             # a piece of one chunk
+    (16, 3000, 72),        # many K splits of one column tile
+    (40, 1096, 200),       # 64-row tile, a partial chunk
+    (130, 584, 392),
+    (300, 2056, 264),      # past the rows that scale x in LDS when aligned
+])
+def test_operands_off_16_byte_boundaries(M, K, N, layout):
+    """Contiguous tensors at any element address, as views of a larger one are."""
+    import yirage_amd.fused as F
+
+    print(f"case unaligned M={M} K={K} N={N} layout={layout}", flush=True)
+    gen = torch.Generator().manual_seed(M + K)
+    dtype = torch.bfloat16 if M % 2 else torch.float16
+    x, (w, w3), gamma, res = _case(M, K, N, layout, dtype, gen)
+    wd, w3d = ((t if layout == KN else t.t()).double() for t in (w, w3))
+    xd = x.double()
+    a = xd @ wd
+    rs = torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    out = _odd(torch.zeros_like(res))
+    xo, wo, w3o, go, ro = (_odd(t) for t in (x, w, w3, gamma, res))
+    for ops in ((xo, wo, ro), (x, wo, res), (xo, w, res)):
+        F.linear(ops[0], ops[1], residual=ops[2], w_layout=layout, out=out)
+        _check(out, a + res.double(), "linear")
+        first = out.clone()
+        F.linear(ops[0], ops[1], residual=ops[2], w_layout=layout, out=out)  # tickets re-armed
+        assert torch.equal(out, first)
+    _check(F.gated_mlp(xo, wo, w3o, w_layout=layout), a * torch.sigmoid(a) * (xd @ w3d), "gated_mlp")
+    _check(F.gated_mlp(x, w, w3o, w_layout=layout), a * torch.sigmoid(a) * (xd @ w3d), "gated_mlp, W3 off")
+    ref = ((x * gamma).double() @ wd) * rs
+    _check(F.rmsnorm_linear(xo, go, wo, w_layout=layout), ref, "rmsnorm_linear")
+    _check(F.rmsnorm_linear(x, go, w, w_layout=layout), ref, "rmsnorm_linear, gamma off")
+    _check(F.rmsnorm_linear(xo, None, w, w_layout=layout), a * rs, "rmsnorm_linear, no gamma")
+
+
 @pytest.mark.parametrize("M", [40, 300])
 def test_special_values_stay_in_their_rows(M):
     """Inf and NaN in one row of x (and none elsewhere) reach that row only:

@@ -1,0 +1,37 @@
+"""Which kernel a call runs on (yr_hip_fused_plan, host only)."""
+import ctypes
+
+import pytest
+
+from yirage_amd import _lib
+
+ONE_ROW, PRODUCT = 0, 1
+
+
+def product_plan(kind, M, K, N, layout, aligned=True):
+    """kernel, rows, columns, splits, row pass, through registers"""
+    p = (ctypes.c_int64 * 6)(M, K, N, _lib.DTYPE_BF16, layout, 0)
+    plan = (ctypes.c_int * 6)()
+    n = 6 if kind == _lib.OP_RMSNORM_LINEAR else 5
+    assert _lib.lib().yr_hip_fused_plan(kind, n, p, int(aligned), plan) == 0, _lib.last_error()
+    return tuple(plan)
+
+
+@pytest.mark.parametrize("kind", [_lib.OP_LINEAR, _lib.OP_RMSNORM_LINEAR, _lib.OP_GATED_MLP])
+@pytest.mark.parametrize("layout", [_lib.W_NK, _lib.W_KN])
+@pytest.mark.parametrize("M,K,N", [(1, 4096, 4096), (16, 3000, 72), (40, 1096, 200), (130, 584, 392),
+                                   (300, 2056, 264), (2048, 4096, 14336)])
+def test_unaligned_operands_pass_through_registers(kind, layout, M, K, N):
+    """Direct loads into LDS need 16-byte aligned operands; others take a tile
+    that loads through registers, within the same workspace."""
+    assert product_plan(kind, M, K, N, layout)[5] == 0
+    kernel, rows, cols, splits, row_pass, staged = product_plan(kind, M, K, N, layout, aligned=False)
+    if kernel == ONE_ROW:  # loads x and W through registers always
+        return
+    assert kernel == PRODUCT and staged == 1 and row_pass == 0 and (rows, cols) in ((32, 128), (64, 128))
+    name = {_lib.OP_LINEAR: "linear", _lib.OP_RMSNORM_LINEAR: "rmsnorm_linear", _lib.OP_GATED_MLP: "gated_mlp"}[kind]
+    have = getattr(_lib.lib(), f"yr_hip_{name}_workspace")(M, K, N, _lib.DTYPE_BF16, layout)
+    if splits > 1:
+        ncol = cols // 2 if kind == _lib.OP_GATED_MLP else cols
+        records = -(-M // rows) * -(-N // ncol) * splits * rows * cols * 4
+        assert 64 * 1024 + records <= have

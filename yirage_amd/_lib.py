@@ -68,6 +68,7 @@ SIGNATURES = {
     "yr_hip_argmax": (_I, [_P, _P, _I, _I, _I, _I, _P]),
     "yr_hip_run_fused": (_I, [_I, _I, _P, _I, _P, _I, _P, _P, _SZ, _P]),
     "yr_hip_fused_workspace": (_SZ, [_I, _I, _P]),
+    "yr_hip_fused_plan": (_I, [_I, _I, _P, _I, _P]),
     "yr_hip_graph_attention_workspace": (_SZ, [_I, _I, _I, _I, _P]),
     "yr_hip_graph_attention": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P, _F, _I, _P, _SZ, _P]),
     "yr_hip_graph_pack": (_I, [_P, _P, _I, _I, _I, _I, _P, _I, _P]),

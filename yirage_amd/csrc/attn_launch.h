@@ -33,6 +33,7 @@ int prefill_launch(const char* nm, const void* q, const void* k, const void* v, 
 bool graph_attn_direct(int G, int M, int L, int d, const long long* sq, const long long* sk, const long long* sv,
                        const long long* so);
 size_t graph_attn_direct_workspace(int G, int M, int L, int d);
+void graph_attn_plan(int G, int M, int L, int d, int* rows_chunk_splits);
 int graph_attn_launch(const char* nm, const void* q, const void* k, const void* v, void* out, int G, int M, int L,
                       int d, const long long* sq, const long long* sk, const long long* sv, const long long* so,
                       float scale, int dtype, void* workspace, hipStream_t st);

@@ -5,6 +5,8 @@
 // runs each one through yr_hip_run_fused on a shared workspace.
 #include <string.h>
 
+#include "attn_launch.h"
+#include "gemm.h"
 #include "yr_common.h"
 
 using namespace yr;
@@ -66,6 +68,29 @@ size_t yr_hip_fused_workspace(int op_kind, int n_params, const int64_t* p) {
     default:
       return 0;
   }
+}
+
+int yr_hip_fused_plan(int op_kind, int n_params, const int64_t* p, int aligned, int* plan6) {
+  const char* nm = "yr_hip_fused_plan";
+  Arity ar;
+  if (!p || !plan6 || !arity_of(op_kind, &ar) || n_params != ar.n_params)
+    return fail(YR_E_INVALID, "%s: op kind %d with %d params", nm, op_kind, n_params);
+  for (int i = 0; i < 6; i++) plan6[i] = 0;
+  if (op_kind == YR_OP_ATTENTION) {
+    const long long* s = reinterpret_cast<const long long*>(p + 6);
+    const int G = (int)p[0], M = (int)p[1], L = (int)p[2], d = (int)p[3];
+    if (G <= 0 || M <= 0 || L <= 0 || d <= 0 || d > 128 || d % 8) return fail(YR_E_INVALID, "%s: shape", nm);
+    plan6[0] = YR_PLAN_PACKED;
+    if (aligned && graph_attn_direct(G, M, L, d, s, s + 3, s + 6, s + 9)) {
+      plan6[0] = YR_PLAN_ATTENTION;
+      graph_attn_plan(G, M, L, d, plan6 + 1);
+    }
+    return YR_OK;
+  }
+  const int epi = op_kind == YR_OP_LINEAR ? 0 : op_kind == YR_OP_RMSNORM_LINEAR ? 1 : op_kind == YR_OP_GATED_MLP ? 2 : -1;
+  if (epi < 0 || !linear_plan(epi, (int)p[0], (int)p[1], (int)p[2], (int)p[4], aligned != 0, plan6))
+    return fail(YR_E_INVALID, "%s: op kind %d has no plan for this shape", nm, op_kind);
+  return YR_OK;
 }
 
 int yr_hip_run_fused(int op_kind, int n_in, const void* const* in, int n_out, void* const* out, int n_params,

@@ -75,8 +75,24 @@ constexpr Cost kCostNorm = {{0.193f, 0.332f, 0.438f},
                         {0.765f, 1.112f, 1.085f},
                         3.12f, 7.08f, 1.25f, 1.039f, 0.067f, 0.250f};
 
-// The best plan of one kind (`pass`: RMSNorm with its row pass) and its time.
-static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* time) {
+// Scratch after the tickets: row factors and scaled x of the row pass, then
+// the records of the K splits.
+static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+static size_t pass_bytes(const Plan& p, int M, int K) {
+  return p.pass ? align256((size_t)M * 4) + align256((size_t)M * K * 2) : 0;
+}
+static size_t split_bytes(int cfg, long tiles, int splits, bool lds_norm) {
+  const CfgShape& s = kCfg[cfg];
+  // one float4 more per thread where a normalising tile also adds row sums
+  const size_t rec = (size_t)s.bm * s.bn * 4 + (lds_norm ? 512 * 16 : 0);
+  return splits > 1 ? (size_t)tiles * splits * rec : 0;
+}
+
+// The best plan of one kind (`pass`: RMSNorm with its row pass) and its time;
+// `staged`: of the tiles that load through registers, with at most `most`
+// bytes of records.
+static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* time, bool staged = false,
+                      size_t most = 0) {
   Plan best = {};
   best.pass = pass;
   const bool lds_norm = epi == EPI_RMSNORM && !pass;
@@ -89,6 +105,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
     if (epi == EPI_GATED && (f == C32x64 || f == C128x192)) continue;
     if (lds_norm && f > C64x128) break;
     if (pass && f <= C64x128) continue;
+    if (staged && f != C32x128 && f != C64x128) continue;
     if (s.bm > 32 && s.bm >= 2 * M && !pass) break;  // a smaller tile holds every row
     if ((size_t)K * 2 * s.bm >= kOob) break;              // 32-bit offsets within a tile's rows of x
     const int tm = (M + s.bm - 1) / s.bm, tn = (N + s.bn / nmat - 1) / (s.bn / nmat);
@@ -103,6 +120,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
       if (sp > 1 && (chunks < 5 * sp || tiles * sp > 4 * kCus || tiles > kMaxTickets)) break;
       const int per = (chunks + sp - 1) / sp;
       if ((chunks + per - 1) / per != sp) continue;
+      if (staged && split_bytes(f, tiles, sp, lds_norm) > most) continue;
       const long wg = tiles * sp, cap = (long)kCus * per_cu, rounds = wg / cap, rest = wg % cap;
       float t = rounds * (per_cu > 1 ? c.chunk_full[f] : c.chunk[f]);
       if (rest) t += rest <= kCus ? c.chunk[f] : c.chunk_full[f];
@@ -132,32 +150,34 @@ static Plan make_plan(int M, int K, int N, int epi, bool nkl) {
   return t0 < t1 ? q : p;
 }
 
+static size_t plan_bytes(const Plan& p, int M, int K, int epi) {
+  const size_t more =
+      pass_bytes(p, M, K) + split_bytes(p.cfg, (long)p.tm * p.tn, p.splits, epi == EPI_RMSNORM && !p.pass);
+  return more ? kTicketBytes + more : 0;
+}
+
+// Operands through registers: no row pass, and no more scratch than the plan
+// for aligned operands has, since the workspace query knows no addresses.
+static Plan make_staged_plan(int M, int K, int N, int epi, bool nkl) {
+  float t;
+  const size_t have = plan_bytes(make_plan(M, K, N, epi, nkl), M, K, epi);
+  return best_plan(M, K, N, epi, nkl, false, &t, true, have ? have - kTicketBytes : 0);
+}
+
 // A plan depends on the sizes alone; a thread keeps the last ones it made
 // (the workspace query and the call ask for the same one).
-static Plan plan(int M, int K, int N, int epi, bool nkl) {
+static Plan plan(int M, int K, int N, int epi, bool nkl, bool staged = false) {
   struct Entry {
     int M, K, N, how;
     Plan p;
   };
   constexpr int kEntries = 64;
   static thread_local Entry kept[kEntries] = {};
-  const int how = 1 + epi * 2 + (nkl ? 1 : 0);
+  const int how = 1 + epi * 2 + (nkl ? 1 : 0) + (staged ? 8 : 0);
   Entry& e = kept[((uint32_t)M * 31 + (uint32_t)K * 7 + (uint32_t)N / 8 + how) % kEntries];
-  if (e.M != M || e.K != K || e.N != N || e.how != how) e = {M, K, N, how, make_plan(M, K, N, epi, nkl)};
+  if (e.M != M || e.K != K || e.N != N || e.how != how) 
+    e = {M, K, N, how, staged ? make_staged_plan(M, K, N, epi, nkl) : make_plan(M, K, N, epi, nkl)};
   return e.p;
-}
-
-static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-// after the tickets: row factors and scaled x of the row pass, then records
-static size_t pass_bytes(const Plan& p, int M, int K) {
-  return p.pass ? align256((size_t)M * 4) + align256((size_t)M * K * 2) : 0;
-}
-static size_t plan_bytes(const Plan& p, int M, int K, int epi) {
-  const CfgShape& s = kCfg[p.cfg];
-  // one float4 more per thread where a normalising tile also adds row sums
-  const size_t rec = (size_t)s.bm * s.bn * 4 + (epi == EPI_RMSNORM && !p.pass ? 512 * 16 : 0);
-  const size_t more = pass_bytes(p, M, K) + (p.splits > 1 ? (size_t)p.tm * p.tn * p.splits * rec : 0);
-  return more ? kTicketBytes + more : 0;
 }
 
 // Column panels: a tile's W rows (N x K) are reached by 32-bit offsets, so K
@@ -181,8 +201,18 @@ size_t workspace(int M, int K, int N, int epi, bool nkl) {
   return need;
 }
 
+void describe(int M, int K, int N, int epi, bool nkl, bool staged, int* plan6) {
+  const int cols = panel_cols(K, N, nkl);
+  const Plan p = plan(M < kPanelRows ? M : kPanelRows, K, N < cols ? N : cols, epi, nkl, staged);
+  const int d[6] = {YR_PLAN_PRODUCT, kCfg[p.cfg].bm, kCfg[p.cfg].bn, p.splits, p.pass, staged};
+  for (int i = 0; i < 6; i++) plan6[i] = d[i];
+}
+
 int run(const Call& c, void* ws, hipStream_t st, const char* name) {
   const int cols = panel_cols(c.K, c.N, c.nkl);
+  // K and N are multiples of 8, so every row and panel keeps the alignment
+  const bool staged =
+      (((uintptr_t)c.x | (uintptr_t)c.gamma | (uintptr_t)c.w0 | (uintptr_t)c.w1) & 15) != 0;
   for (int m0 = 0; m0 < c.M; m0 += kPanelRows)
     for (int n0 = 0; n0 < c.N; n0 += cols) {
       Args a = {};
@@ -190,7 +220,7 @@ int run(const Call& c, void* ws, hipStream_t st, const char* name) {
       a.K = c.K;
       a.N = c.N - n0 < cols ? c.N - n0 : cols;
       a.ldo = c.N;
-      const Plan p = plan(a.M, a.K, a.N, c.epi, c.nkl);
+      const Plan p = plan(a.M, a.K, a.N, c.epi, c.nkl, staged);
       a.x = c.x + (size_t)m0 * c.K;
       a.gamma = c.gamma;
       a.w0 = c.w0 + (size_t)n0 * c.K;  // n0 > 0 only for N x K weights
@@ -216,9 +246,9 @@ int run(const Call& c, void* ws, hipStream_t st, const char* name) {
         if (c.gamma) a.x = xg;
       }
       a.partial = (float*)(scratch + pass_bytes(p, a.M, a.K));
-      if (c.epi == EPI_GATED) launch<EPI_GATED>(p.cfg, c.dtype, c.nkl, a, st);
-      else if (c.epi == EPI_RMSNORM) launch<EPI_RMSNORM>(p.cfg, c.dtype, c.nkl, a, st);
-      else launch<EPI_LINEAR>(p.cfg, c.dtype, c.nkl, a, st);
+      if (c.epi == EPI_GATED) launch<EPI_GATED>(p.cfg, c.dtype, c.nkl, staged, a, st);
+      else if (c.epi == EPI_RMSNORM) launch<EPI_RMSNORM>(p.cfg, c.dtype, c.nkl, staged, a, st);
+      else launch<EPI_LINEAR>(p.cfg, c.dtype, c.nkl, staged, a, st);
       YR_CHECK_LAUNCH(name);
     }
   return YR_OK;

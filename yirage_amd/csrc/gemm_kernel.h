@@ -22,6 +22,11 @@
 // of the loads (the LDS image of one load instruction is contiguous), so that
 // fragment reads are free of bank conflicts: 128-byte rows (x, and W in
 // N x K) by row % 8, K x N rows of 128 or 64 columns by w_swz.
+//
+// Direct loads need 16-byte aligned operands.  Without DMA (x, gamma or W at
+// another address) the same pieces pass through registers: the loads of a
+// chunk are issued where the direct ones are, and written to the stage one
+// chunk later, behind the next barrier.
 #pragma once
 #include <type_traits>
 
@@ -132,7 +137,7 @@ __device__ __forceinline__ float sumsq8(uint4 x, float s) {
 // WM x WN waves; wave (wm, wn) owns rows wm BM / WM .. of the tile and
 // BN / WN columns (for the gated MLP the same BN / WN / 2 columns of both
 // matrices, so its lanes hold both factors of an output).
-template <int DT, int EPI, bool NKL, int BM, int BN, int WM, int WN, int NST>
+template <int DT, int EPI, bool NKL, int BM, int BN, int WM, int WN, int NST, bool DMA>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
   constexpr bool NORM = EPI == EPI_RMSNORM_LDS;
   constexpr int NW = WM * WN, NMAT = EPI == EPI_GATED ? 2 : 1, BNM = BN / NMAT;
@@ -144,7 +149,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
   static_assert(XB % (1024 * NW) == 0 && MB % (1024 * NW) == 0, "whole loads per wave");
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, NJM = NJ / NMAT;  // MFMA blocks per wave
   constexpr int SW = BNM % 128 == 0 ? 128 : 64;                         // K x N: columns of a sub-tile
-  static_assert(BNM % SW == 0 && NST >= (NORM ? 3 : 2) && (NST - 1) * LPW < 64, "stages");
+  static_assert(BNM % SW == 0 && NST >= (NORM ? 3 : 2) + (DMA ? 0 : 1) && (NST - 1) * LPW < 64, "stages");
   constexpr int NP = NORM ? BM * 8 / (64 * NW) : 1;                     // 16-byte pieces of x per thread and chunk
   static_assert(!NORM || (NP >= 1 && BM * 8 % (64 * NW) == 0), "whole pieces per thread");
   __shared__ __attribute__((aligned(16))) char lds[NST * (XB + WB + GB)];  // x stages, W stages, gamma stages
@@ -223,6 +228,45 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
       }
       if constexpr (NORM)
         bload_lds16(rg, 8 * lane < krel ? (uint32_t)((kbeg + ci * KS + 8 * lane) * 2) : kOob, 0, gd + s * GB);
+    }
+  };
+
+  // without DMA: the pieces of chunk ci into registers (global loads, any
+  // address), and from there into stage s
+  uint4 held[DMA ? 1 : LPW];
+  auto hold = [&](int ci) __attribute__((always_inline)) {
+    const int krel = kend - kbeg - ci * KS;
+    const uint4 zero = make_uint4(0, 0, 0, 0);
+    if (krel <= 0) return;
+#pragma unroll
+    for (int p = 0; p < LPW; p++) {
+      const char* base;
+      uint32_t off;
+      int k;
+      if (p < NX) {
+        base = reinterpret_cast<const char*>(a.x + (size_t)m0 * a.K);
+        off = xo[p < NX ? p : 0] + (uint32_t)ci * (KS * 2);
+        k = 8 * pchunk;
+      } else if (p < NX + NWL) {
+        const int i = p - NX;
+        base = reinterpret_cast<const char*>((i < NBM / NW ? a.w0 : a.w1) + wbase);
+        off = wo[i] + (uint32_t)ci * wstep;
+        k = NKL ? 8 * pchunk : RPB * (((wave + NW * i) % NBM) % BPS) + lane / CPR;
+      } else {
+        base = reinterpret_cast<const char*>(a.gamma);
+        off = (uint32_t)((kbeg + ci * KS + 8 * lane) * 2);
+        k = lane < 8 && a.gamma ? 8 * lane : KS;
+      }
+      held[DMA ? 0 : p] = k < min(krel, KS) ? ldg16(base + off) : zero;
+    }
+  };
+  auto put_held = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < LPW; p++) {
+      const uint32_t d = p < NX        ? xd + s * XB + 1024 * NW * p
+                         : p < NX + NWL ? wd + s * WB + 1024 * NW * (p - NX)
+                                        : gd + s * GB;
+      *reinterpret_cast<uint4*>(lds + (d - lds0) + 16 * lane) = held[DMA ? 0 : p];
     }
   };
 
@@ -328,7 +372,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
     else wait_and_sync<0>();
     if constexpr (NORM)
       if (LD || ci + 2 < nch) norm_rd(s2);
-    if constexpr (!LD) issue(ci + NST, s);
+    if constexpr (!DMA) {  // chunk ci - 1 + NST has come in since the last barrier
+      if (ci > 0 && ci - 1 + NST < nch) put_held((s + NST - 1) % NST);
+      hold(ci + NST);
+    } else if constexpr (!LD) {
+      issue(ci + NST, s);
+    }
     half(f1, f0, 0, s1, ldc, ci + NST, s);
   };
   auto round = [&](int ci, auto self, auto sc, auto ldc) __attribute__((always_inline)) {
@@ -337,7 +386,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
     if constexpr (s + 1 < NST) self(ci, self, std::integral_constant<int, s + 1>{}, ldc);
   };
 #pragma unroll
-  for (int c = 0; c < NST; c++) issue(c, c);
+  for (int c = 0; c < NST; c++) {
+    if constexpr (DMA) {
+      issue(c, c);
+    } else if (c < nch) {
+      hold(c);
+      put_held(c);
+    }
+  }
   if (nch >= NST) wait_and_sync<(NST - AHEAD) * LPW>();
   else wait_and_sync<0>();
   if constexpr (NORM) {
@@ -357,7 +413,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Args a) {
   for (int i = 0; i < MI; i++) f0.x[i] = rd_x(i, 0, 0);
   int ci = 0;
   const int nwhole = (kend - kbeg) / KS;
-  for (; ci + 2 * NST <= nwhole; ci += NST) round(ci, round, std::integral_constant<int, 0>{}, std::true_type{});
+  for (; DMA && ci + 2 * NST <= nwhole; ci += NST) round(ci, round, std::integral_constant<int, 0>{}, std::true_type{});
   for (; ci < nch; ci += NST) round(ci, round, std::integral_constant<int, 0>{}, std::false_type{});
 
   // RMSNorm in LDS: a row's sum is with the 8 lanes of its pieces

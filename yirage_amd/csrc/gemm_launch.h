@@ -6,9 +6,9 @@
 namespace yr {
 namespace gm {
 
-template <int DT, int EPI, bool NKL, int BM, int BN, int WM, int WN, int NST>
+template <int DT, int EPI, bool NKL, int BM, int BN, int WM, int WN, int NST, bool DMA = true>
 static void go(const Args& a, hipStream_t st) {
-  hipLaunchKernelGGL((gemm_kernel<DT, EPI, NKL, BM, BN, WM, WN, NST>), dim3(a.tm * a.tn * a.splits),
+  hipLaunchKernelGGL((gemm_kernel<DT, EPI, NKL, BM, BN, WM, WN, NST, DMA>), dim3(a.tm * a.tn * a.splits),
                      dim3(64 * WM * WN), 0, st, a);
 }
 
@@ -46,15 +46,29 @@ static void go_cfg(int cfg, const Args& a, hipStream_t st) {
   }
 }
 
+// Operands that are not 16-byte aligned: two tiles, both of which also scale x
+// themselves; the loads through registers want a stage more than direct ones.
+// One chunk per workgroup in flight bounds them: 8 rows, 4096 x 4096 20 us
+// (12 aligned), 128 rows, 4096 x 14336 51 us (29), 2048 rows, 4096 x 4096 186
+// us (61).
+template <int DT, int EPI, bool NKL>
+static void go_staged(int cfg, const Args& a, hipStream_t st) {
+  constexpr int E = EPI == EPI_RMSNORM ? EPI_RMSNORM_LDS : EPI;
+  if (cfg == C32x128) go<DT, E, NKL, 32, 128, 1, 4, EPI == EPI_RMSNORM ? 4 : 3, false>(a, st);
+  else go<DT, E, NKL, 64, 128, 2, 4, 6, false>(a, st);
+}
+
 template <int EPI>
-void launch(int cfg, int dtype, bool nkl, const Args& a, hipStream_t st) {
-  if (dtype == YR_DTYPE_F16) {
-    if (nkl) go_cfg<DT_F16, EPI, true>(cfg, a, st);
-    else go_cfg<DT_F16, EPI, false>(cfg, a, st);
-  } else {
-    if (nkl) go_cfg<DT_BF16, EPI, true>(cfg, a, st);
-    else go_cfg<DT_BF16, EPI, false>(cfg, a, st);
-  }
+void launch(int cfg, int dtype, bool nkl, bool staged, const Args& a, hipStream_t st) {
+  auto run = [&](auto dt, auto nk) {
+    constexpr int DT = decltype(dt)::value;
+    constexpr bool NKL = decltype(nk)::value;
+    if (staged) go_staged<DT, EPI, NKL>(cfg, a, st);
+    else go_cfg<DT, EPI, NKL>(cfg, a, st);
+  };
+  auto with = [&](auto dt) { nkl ? run(dt, std::true_type{}) : run(dt, std::false_type{}); };
+  if (dtype == YR_DTYPE_F16) with(std::integral_constant<int, DT_F16>{});
+  else with(std::integral_constant<int, DT_BF16>{});
 }
 
 }  // namespace gm

@@ -389,6 +389,13 @@ bool graph_attn_direct(int G, int M, int L, int d, const long long* sq, const lo
 
 size_t graph_attn_direct_workspace(int G, int M, int L, int d) { return kTicketBytes + ga::plan(G, M, L, d).bytes; }
 
+void graph_attn_plan(int G, int M, int L, int d, int* rows_chunk_splits) {
+  const ga::Plan p = ga::plan(G, M, L, d);
+  rows_chunk_splits[0] = 16 << p.cfg;
+  rows_chunk_splits[1] = p.chunk;
+  rows_chunk_splits[2] = p.splits;
+}
+
 int graph_attn_launch(const char* nm, const void* q, const void* k, const void* v, void* out, int G, int M, int L,
                       int d, const long long* sq, const long long* sk, const long long* sv, const long long* so,
                       float scale, int dtype, void* workspace, hipStream_t st) {

@@ -160,12 +160,26 @@ static size_t gemv_workspace(int K, int N, int nmat) {
   return slices > 1 ? kTicketBytes + tiles * slices * round_up4(nmat * NK_TROWS + 1) * sizeof(float) : 0;
 }
 
+static bool ws_ok(int B, int K, int N) { return B > 0 && K > 0 && N > 0 && (size_t)K * 2 * 32 < kOob; }
+
 static size_t ws_for(int B, int K, int N, int layout, int epi) {
-  if (B <= 0 || K <= 0 || N <= 0 || (size_t)K * 2 * 32 >= kOob) return 0;
+  if (!ws_ok(B, K, N)) return 0;
   if (one_row(B, K, N, layout, epi)) return gemv_workspace(K, N, epi == EPI_GATED ? 2 : 1);
   const size_t w = gm::workspace(B, K, N, epi, layout == YR_W_NK);
   // K x N calls hold the ticket region at least, whether or not K is split
   return layout == YR_W_KN && w < kTicketBytes ? kTicketBytes : w;
+}
+
+// The launch of a call (yr_hip_fused_plan).
+bool linear_plan(int epi, int B, int K, int N, int layout, bool aligned, int* plan6) {
+  if (!ws_ok(B, K, N) || K % 8 || N % 8) return false;
+  if (one_row(B, K, N, layout, epi)) {
+    const int d[6] = {YR_PLAN_ONE_ROW, 1, NK_TROWS, (K + NK_SLICE - 1) / NK_SLICE, 0, 0};
+    for (int i = 0; i < 6; i++) plan6[i] = d[i];
+  } else {
+    gm::describe(B, K, N, epi, layout == YR_W_NK, !aligned, plan6);
+  }
+  return true;
 }
 
 template <int NMAT, int EPI>
