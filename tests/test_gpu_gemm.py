@@ -151,3 +151,26 @@ def test_n_by_k_weights_past_4_gib():
     out = F.linear(x, w)
     for cols in (slice(0, 72), slice(N - 72, N)):
         _check(out[:, cols], x.double() @ w[cols].double().t(), "linear")
+
+
+@pytest.mark.parametrize("M,layout", [(1, NK), (3, KN), (17, NK)])
+def test_long_k(M, layout):
+    """K = 2^26: few rows and columns, operands below 4 GiB."""
+    import yirage_amd.fused as F
+
+    K, N = 1 << 26, 8
+    print(f"case long K M={M} layout={layout}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.empty((M, K), dtype=torch.bfloat16, device="cuda").normal_(generator=gen)
+    w = torch.empty((K, N) if layout == KN else (N, K), dtype=torch.bfloat16, device="cuda")
+    w.normal_(0.0, K ** -0.5, generator=gen)
+    ref = torch.zeros((M, N), dtype=torch.float64, device="cuda")
+    ss = torch.zeros((M, 1), dtype=torch.float64, device="cuda")
+    for k in range(0, K, 1 << 22):
+        xd = x[:, k:k + (1 << 22)].double()
+        ref += xd @ (w[k:k + (1 << 22)] if layout == KN else w[:, k:k + (1 << 22)].t()).double()
+        ss += (xd * xd).sum(-1, keepdim=True)
+    # fp32 sums in chunks: each of the K / 64 chunk sums adds at most half an
+    # ulp of the running sum (about 1): 2^20 2^-24 at worst, 2^10 2^-24 at random
+    _check(F.linear(x, w, w_layout=layout), ref, "linear")
+    _check(F.rmsnorm_linear(x, None, w, w_layout=layout), ref * torch.rsqrt(ss / K + 1e-6), "rmsnorm_linear")

@@ -35,3 +35,18 @@ def test_unaligned_operands_pass_through_registers(kind, layout, M, K, N):
         ncol = cols // 2 if kind == _lib.OP_GATED_MLP else cols
         records = -(-M // rows) * -(-N // ncol) * splits * rows * cols * 4
         assert 64 * 1024 + records <= have
+
+
+@pytest.mark.parametrize("kind", [_lib.OP_LINEAR, _lib.OP_RMSNORM_LINEAR, _lib.OP_GATED_MLP])
+def test_longest_k(kind):
+    """K of 2^26 and more while the rows of x and the weights stay below 4 GiB;
+    one row on N x K weights as far as the one-row kernel's grid reaches."""
+    K = 1 << 26
+    for M, N, layout, kernel in ((1, 8, _lib.W_NK, ONE_ROW), (1, 8, _lib.W_KN, PRODUCT), (3, 16, _lib.W_KN, PRODUCT),
+                                 (31, 8, _lib.W_KN, PRODUCT), (20, 8, _lib.W_NK, PRODUCT)):
+        assert product_plan(kind, M, K, N, layout)[0] == kernel
+    assert product_plan(kind, 1, 65535 * 2048, 8, _lib.W_NK)[0] == ONE_ROW
+    for M, k, layout in ((2, K, _lib.W_NK), (32, K, _lib.W_KN), (1, 65536 * 2048, _lib.W_NK)):
+        p = (ctypes.c_int64 * 6)(M, k, 8, _lib.DTYPE_BF16, layout, 0)
+        n = 6 if kind == _lib.OP_RMSNORM_LINEAR else 5
+        assert _lib.lib().yr_hip_fused_plan(kind, n, p, 1, (ctypes.c_int * 6)()) != 0

@@ -107,7 +107,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
     if (pass && f <= C64x128) continue;
     if (staged && f != C32x128 && f != C64x128) continue;
     if (s.bm > 32 && s.bm >= 2 * M && !pass) break;  // a smaller tile holds every row
-    if ((size_t)K * 2 * s.bm >= kOob) break;              // 32-bit offsets within a tile's rows of x
+    if ((size_t)K * 2 * (M < s.bm ? M : s.bm) >= kOob) break;  // 32-bit offsets within a tile's rows of x
     const int tm = (M + s.bm - 1) / s.bm, tn = (N + s.bn / nmat - 1) / (s.bn / nmat);
     const long tiles = (long)tm * tn;
     // two workgroups per CU need two times their LDS: the normalising 32 x

@@ -149,8 +149,11 @@ __global__ __launch_bounds__(NK_THREADS) void gemv_nk_kernel(GemvArgs a) {
 //   linear  2048 x 2048 4.2 / 5.7, 2048 x 8192 7.5 / 7.2, 4096 x 1024 5.9 / 6.6,
 //           4096 x 4096 9.5 / 8.8
 //   gated   2048 x 4096 8.5 / 9.2, 2048 x 8192 12.7 / 11.7, 3072 x 2048 9.6 / 8.9
+constexpr int kLongK = 1 << 26;  // 32 rows of x reach 4 GiB
+
 static bool one_row(int B, int K, int N, int layout, int epi) {
   if (B != 1 || layout != YR_W_NK) return false;
+  if (K >= kLongK) return true;  // the product kernel cuts K in 16 at most, this one in any number of slices
   if (K <= NK_SLICE) return epi == EPI_RMSNORM || N <= 6144;
   return epi != EPI_GATED && (long long)K * N <= (epi == EPI_RMSNORM ? 1ll << 23 : 1ll << 22);
 }
@@ -160,10 +163,18 @@ static size_t gemv_workspace(int K, int N, int nmat) {
   return slices > 1 ? kTicketBytes + tiles * slices * round_up4(nmat * NK_TROWS + 1) * sizeof(float) : 0;
 }
 
-static bool ws_ok(int B, int K, int N) { return B > 0 && K > 0 && N > 0 && (size_t)K * 2 * 32 < kOob; }
+// K a kernel takes: the product kernel reaches the (up to 32) rows of x of its
+// smallest tile by 32-bit offsets, 2..16 rows on N x K weights end at 2^26, and
+// the one-row kernel at the K slices that its grid can hold.
+static bool k_fits(int B, int K, int layout) {
+  if (layout == YR_W_NK && B == 1) return K <= 65535ll * NK_SLICE;
+  if (layout == YR_W_NK && B <= 16 && K >= kLongK) return false;
+  return (size_t)K * 2 * (B < 32 ? B : 32) < kOob;
+}
+static bool ws_ok(int B, int K, int N, int layout) { return B > 0 && K > 0 && N > 0 && k_fits(B, K, layout); }
 
 static size_t ws_for(int B, int K, int N, int layout, int epi) {
-  if (!ws_ok(B, K, N)) return 0;
+  if (!ws_ok(B, K, N, layout)) return 0;
   if (one_row(B, K, N, layout, epi)) return gemv_workspace(K, N, epi == EPI_GATED ? 2 : 1);
   const size_t w = gm::workspace(B, K, N, epi, layout == YR_W_NK);
   // K x N calls hold the ticket region at least, whether or not K is split
@@ -172,7 +183,7 @@ static size_t ws_for(int B, int K, int N, int layout, int epi) {
 
 // The launch of a call (yr_hip_fused_plan).
 bool linear_plan(int epi, int B, int K, int N, int layout, bool aligned, int* plan6) {
-  if (!ws_ok(B, K, N) || K % 8 || N % 8) return false;
+  if (!ws_ok(B, K, N, layout) || K % 8 || N % 8) return false;
   if (one_row(B, K, N, layout, epi)) {
     const int d[6] = {YR_PLAN_ONE_ROW, 1, NK_TROWS, (K + NK_SLICE - 1) / NK_SLICE, 0, 0};
     for (int i = 0; i < 6; i++) plan6[i] = d[i];
@@ -200,8 +211,8 @@ static int run_linear(GemvArgs a, int dtype, int layout, void* ws, size_t ws_byt
   const size_t xrows = layout == YR_W_KN || a.B < 128 ? a.B : 128;
   if ((layout == YR_W_KN || a.B > 16) && ((size_t)a.K * a.N * 2 >= kOob || xrows * a.K * 2 >= kOob))
     return fail(YR_E_INVALID, "%s: operands must be < 4 GiB (32-bit buffer offsets)", name);
+  if (!k_fits(a.B, a.K, layout)) return fail(YR_E_INVALID, "%s: K=%d too large", name, a.K);
   if (!one_row(a.B, a.K, a.N, layout, EPI)) {
-    if ((size_t)a.K * 2 * 32 >= kOob) return fail(YR_E_INVALID, "%s: K=%d too large", name, a.K);
     const gm::Call c = {a.x, a.gamma, a.w0, a.w1, a.residual, a.out, a.B, a.K, a.N, dtype, EPI, layout == YR_W_NK,
                         a.eps};
     return gm::run(c, ws, st, name);
