@@ -50,3 +50,17 @@ def test_longest_k(kind):
         p = (ctypes.c_int64 * 6)(M, k, 8, _lib.DTYPE_BF16, layout, 0)
         n = 6 if kind == _lib.OP_RMSNORM_LINEAR else 5
         assert _lib.lib().yr_hip_fused_plan(kind, n, p, 1, (ctypes.c_int * 6)()) != 0
+
+
+def test_product_scratch_is_bounded():
+    """The workspace of a stream lives as long as the process: 64 MiB of K-split
+    records and 64 MiB for the row pass's copy of x, whatever the shape."""
+    lib = _lib.lib()
+    most = 64 * 1024 + 2 * (64 << 20) + 4 * 8192 + 512
+    for M in (256, 257, 700, 1110, 1654, 2048, 4096, 8192, 8193, 20000):
+        for K in (1024, 4096, 6648, 13984, 14336, 28672, 1 << 18):
+            for N in (256, 3376, 4096, 7744, 11848, 14336):
+                for layout in (_lib.W_NK, _lib.W_KN):
+                    for kind in ("linear", "rmsnorm_linear", "gated_mlp"):
+                        b = getattr(lib, f"yr_hip_{kind}_workspace")(M, K, N, _lib.DTYPE_F16, layout)
+                        assert b <= most, (kind, M, K, N, layout, b)

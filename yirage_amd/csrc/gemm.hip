@@ -48,7 +48,11 @@ constexpr int kCus = 256;
 // pass; 174 rows, K 2928, N 14280: 58.4 against 31.9).
 constexpr int kNormLdsAlways = 64, kNormLdsMax = 256;
 constexpr float kRowPassUs = 3.f;  // a row pass and the gap behind it
-constexpr int kPanelRows = 8192;   // rows per launch: bounds the row pass's copy of x
+constexpr int kPanelRows = 8192;   // rows per launch
+// A stream keeps the largest workspace it has needed, so scratch is bounded:
+// the row pass's copy of x (fewer rows per launch where K is long) and the
+// records of the K splits (one per CU of the largest tile).
+constexpr size_t kPassBytes = 64u << 20, kSplitBytes = 64u << 20;
 
 // Microseconds of one 64-k chunk of a tile, alone on its CU and with as many
 // workgroups per CU as fit, its factor for K x N weights, and the terms around
@@ -120,7 +124,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
       if (sp > 1 && (chunks < 5 * sp || tiles * sp > 4 * kCus || tiles > kMaxTickets)) break;
       const int per = (chunks + sp - 1) / sp;
       if ((chunks + per - 1) / per != sp) continue;
-      if (staged && split_bytes(f, tiles, sp, lds_norm) > most) continue;
+      if (split_bytes(f, tiles, sp, lds_norm) > (staged ? most : kSplitBytes)) continue;
       const long wg = tiles * sp, cap = (long)kCus * per_cu, rounds = wg / cap, rest = wg % cap;
       float t = rounds * (per_cu > 1 ? c.chunk_full[f] : c.chunk[f]);
       if (rest) t += rest <= kCus ? c.chunk[f] : c.chunk_full[f];
@@ -143,7 +147,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
 
 static Plan make_plan(int M, int K, int N, int epi, bool nkl) {
   float t0 = 0.f, t1 = 0.f;
-  if (epi != EPI_RMSNORM || M <= kNormLdsAlways) return best_plan(M, K, N, epi, nkl, false, &t0);
+  if (epi != EPI_RMSNORM || M <= kNormLdsAlways || (size_t)M * K * 2 > kPassBytes) return best_plan(M, K, N, epi, nkl, false, &t0);
   const Plan p = best_plan(M, K, N, epi, nkl, true, &t1);
   if (M > kNormLdsMax) return p;
   const Plan q = best_plan(M, K, N, epi, nkl, false, &t0);
@@ -188,11 +192,19 @@ static int panel_cols(int K, int N, bool nkl) {
   return n < 8 ? 8 : n < N ? n : N;
 }
 
+// Rows per launch: as many as the row pass's copy of x may have (whole 256-row
+// tiles; beyond K = 131072 not even those, and the tiles scale x themselves).
+static int panel_rows(int K, int epi) {
+  if (epi != EPI_RMSNORM) return kPanelRows;
+  const size_t n = kPassBytes / (2 * (size_t)K) / 256 * 256;
+  return n < 256 ? 256 : n < kPanelRows ? (int)n : kPanelRows;
+}
+
 size_t workspace(int M, int K, int N, int epi, bool nkl) {
-  const int cols = panel_cols(K, N, nkl);
+  const int cols = panel_cols(K, N, nkl), most = panel_rows(K, epi);
   size_t need = 0;
   // whole panels are alike: the first one and the remainder
-  for (int rows : {M < kPanelRows ? M : kPanelRows, M % kPanelRows})
+  for (int rows : {M < most ? M : most, M % most})
     for (int nc : {cols, N % cols})
       if (rows > 0 && nc > 0) {
         const size_t b = plan_bytes(plan(rows, K, nc, epi, nkl), rows, K, epi);
@@ -203,20 +215,21 @@ size_t workspace(int M, int K, int N, int epi, bool nkl) {
 
 void describe(int M, int K, int N, int epi, bool nkl, bool staged, int* plan6) {
   const int cols = panel_cols(K, N, nkl);
-  const Plan p = plan(M < kPanelRows ? M : kPanelRows, K, N < cols ? N : cols, epi, nkl, staged);
+  const int most = panel_rows(K, epi);
+  const Plan p = plan(M < most ? M : most, K, N < cols ? N : cols, epi, nkl, staged);
   const int d[6] = {YR_PLAN_PRODUCT, kCfg[p.cfg].bm, kCfg[p.cfg].bn, p.splits, p.pass, staged};
   for (int i = 0; i < 6; i++) plan6[i] = d[i];
 }
 
 int run(const Call& c, void* ws, hipStream_t st, const char* name) {
-  const int cols = panel_cols(c.K, c.N, c.nkl);
+  const int cols = panel_cols(c.K, c.N, c.nkl), most = panel_rows(c.K, c.epi);
   // K and N are multiples of 8, so every row and panel keeps the alignment
   const bool staged =
       (((uintptr_t)c.x | (uintptr_t)c.gamma | (uintptr_t)c.w0 | (uintptr_t)c.w1) & 15) != 0;
-  for (int m0 = 0; m0 < c.M; m0 += kPanelRows)
+  for (int m0 = 0; m0 < c.M; m0 += most)
     for (int n0 = 0; n0 < c.N; n0 += cols) {
       Args a = {};
-      a.M = c.M - m0 < kPanelRows ? c.M - m0 : kPanelRows;
+      a.M = c.M - m0 < most ? c.M - m0 : most;
       a.K = c.K;
       a.N = c.N - n0 < cols ? c.N - n0 : cols;
       a.ldo = c.N;
