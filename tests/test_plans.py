@@ -54,9 +54,9 @@ def test_longest_k(kind):
 
 def test_product_scratch_is_bounded():
     """The workspace of a stream lives as long as the process: 64 MiB of K-split
-    records and 64 MiB for the row pass's copy of x, whatever the shape."""
+    records and 128 MiB for the row pass's copy of x, whatever the shape."""
     lib = _lib.lib()
-    most = 64 * 1024 + 2 * (64 << 20) + 4 * 8192 + 512
+    most = 64 * 1024 + (64 << 20) + (128 << 20) + 4 * 8192 + 512
     for M in (256, 257, 700, 1110, 1654, 2048, 4096, 8192, 8193, 20000):
         for K in (1024, 4096, 6648, 13984, 14336, 28672, 1 << 18):
             for N in (256, 3376, 4096, 7744, 11848, 14336):

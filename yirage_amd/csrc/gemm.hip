@@ -52,7 +52,10 @@ constexpr int kPanelRows = 8192;   // rows per launch
 // A stream keeps the largest workspace it has needed, so scratch is bounded:
 // the row pass's copy of x (fewer rows per launch where K is long) and the
 // records of the K splits (one per CU of the largest tile).
-constexpr size_t kPassBytes = 64u << 20, kSplitBytes = 64u << 20;
+// Records past 64 MiB were no gain either (1654 rows, RMSNorm 6648 x 11848: 379
+// us with two splits of 256 x 256 tiles, 318 without; 1730 rows, gated 14192 x
+// 3376: 403 with four, 280 without).
+constexpr size_t kPassBytes = 128u << 20, kSplitBytes = 64u << 20;
 
 // Microseconds of one 64-k chunk of a tile, alone on its CU and with as many
 // workgroups per CU as fit, its factor for K x N weights, and the terms around
@@ -192,16 +195,19 @@ static int panel_cols(int K, int N, bool nkl) {
   return n < 8 ? 8 : n < N ? n : N;
 }
 
-// Rows per launch: as many as the row pass's copy of x may have (whole 256-row
-// tiles; beyond K = 131072 not even those, and the tiles scale x themselves).
-static int panel_rows(int K, int epi) {
+// Rows per launch.  RMSNorm: as many as the row pass's copy of x may have, in
+// even panels of whole 256-row tiles (beyond K = 262144 not even one tile's
+// rows may, and the tiles scale x themselves).
+static int panel_rows(int M, int K, int epi) {
   if (epi != EPI_RMSNORM) return kPanelRows;
-  const size_t n = kPassBytes / (2 * (size_t)K) / 256 * 256;
-  return n < 256 ? 256 : n < kPanelRows ? (int)n : kPanelRows;
+  int most = (int)(kPassBytes / (2 * (size_t)K)) / 256 * 256;
+  most = most < 256 ? 256 : most < kPanelRows ? most : kPanelRows;
+  const int panels = (M + most - 1) / most;
+  return ((M + panels - 1) / panels + 255) / 256 * 256;
 }
 
 size_t workspace(int M, int K, int N, int epi, bool nkl) {
-  const int cols = panel_cols(K, N, nkl), most = panel_rows(K, epi);
+  const int cols = panel_cols(K, N, nkl), most = panel_rows(M, K, epi);
   size_t need = 0;
   // whole panels are alike: the first one and the remainder
   for (int rows : {M < most ? M : most, M % most})
@@ -215,14 +221,14 @@ size_t workspace(int M, int K, int N, int epi, bool nkl) {
 
 void describe(int M, int K, int N, int epi, bool nkl, bool staged, int* plan6) {
   const int cols = panel_cols(K, N, nkl);
-  const int most = panel_rows(K, epi);
+  const int most = panel_rows(M, K, epi);
   const Plan p = plan(M < most ? M : most, K, N < cols ? N : cols, epi, nkl, staged);
   const int d[6] = {YR_PLAN_PRODUCT, kCfg[p.cfg].bm, kCfg[p.cfg].bn, p.splits, p.pass, staged};
   for (int i = 0; i < 6; i++) plan6[i] = d[i];
 }
 
 int run(const Call& c, void* ws, hipStream_t st, const char* name) {
-  const int cols = panel_cols(c.K, c.N, c.nkl), most = panel_rows(c.K, c.epi);
+  const int cols = panel_cols(c.K, c.N, c.nkl), most = panel_rows(c.M, c.K, c.epi);
   // K and N are multiples of 8, so every row and panel keeps the alignment
   const bool staged =
       (((uintptr_t)c.x | (uintptr_t)c.gamma | (uintptr_t)c.w0 | (uintptr_t)c.w1) & 15) != 0;
