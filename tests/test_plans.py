@@ -64,3 +64,19 @@ def test_product_scratch_is_bounded():
                     for kind in ("linear", "rmsnorm_linear", "gated_mlp"):
                         b = getattr(lib, f"yr_hip_{kind}_workspace")(M, K, N, _lib.DTYPE_F16, layout)
                         assert b <= most, (kind, M, K, N, layout, b)
+
+
+def test_few_rows_of_rmsnorm_fill_the_chip():
+    """Up to 16 rows are bound by the weights: the CU with the most workgroups
+    has at most half as many again as the average one."""
+    worst, total, n = 0.0, 0.0, 0
+    for K in (2048, 3072, 4096, 5120, 8192, 11264):
+        for N in (2048, 3072, 4096, 5120, 6144, 7168, 8192, 9216, 10240, 11264, 14336):
+            if K * N * 2 < 16 << 20:
+                continue
+            for M in (1, 8, 16):
+                _, _, cols, splits, _, _ = product_plan(_lib.OP_RMSNORM_LINEAR, M, K, N, _lib.W_KN)
+                groups = -(-N // cols) * splits
+                uneven = -(-groups // 256) * 256 / groups
+                worst, total, n = max(worst, uneven), total + uneven, n + 1
+    assert worst <= 1.5 and total / n <= 1.2

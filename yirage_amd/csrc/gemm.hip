@@ -45,9 +45,11 @@ constexpr int kCus = 256;
 // RMSNorm: the tiles of up to 64 rows scale x in LDS; up to 64 rows that is
 // always the faster way, beyond 256 rows never, between them the cheaper by
 // the model below (71 rows, K 2992, N 3728: 14.9 us against 18.7 with the row
-// pass; 174 rows, K 2928, N 14280: 58.4 against 31.9).
+// pass; 174 rows, K 2928, N 14280: 58.4 against 31.9).  The row pass counts
+// with what such a call takes beyond the model's time for its product (741
+// shapes of 65..315 rows, least squares): 6.3 us and its two streams of x.
 constexpr int kNormLdsAlways = 64, kNormLdsMax = 256;
-constexpr float kRowPassUs = 3.f;  // a row pass and the gap behind it
+constexpr float kRowPassUs = 6.3f, kRowPassTbs = 1.1f;
 constexpr int kPanelRows = 8192;   // rows per launch
 // A stream keeps the largest workspace it has needed, so scratch is bounded:
 // the row pass's copy of x (fewer rows per launch where K is long) and the
@@ -60,11 +62,11 @@ constexpr size_t kPassBytes = 128u << 20, kSplitBytes = 64u << 20;
 // Microseconds of one 64-k chunk of a tile, alone on its CU and with as many
 // workgroups per CU as fit, its factor for K x N weights, and the terms around
 // it: start, memory TB/s, a K split's merge (fixed, per 64 KB of records, per
-// split) and the slowdown of a full chip.  Fitted to 20,000 timings (390
-// shapes of 1..2048 rows, K and N 1024..14336, every tile and split count).
-// The model only ranks: over those shapes the plan it picks is on average
-// 0.8 % (linear), 0.9 % (gated) and 0.6 % (RMSNorm in LDS) slower than the
-// fastest, 17 % at worst.
+// split) and the slowdown of a full chip.  The model only ranks.  Linear and
+// gated are fitted to calls that repeat their weights, which partly stay in the
+// cache; where the weights come from HBM the plan is on average 3.9 % (linear,
+// 1176 shapes of 2..2048 rows, K and N 720..14264) and 4.0 % (gated, 2007)
+// slower than the fastest, 18 and 17 % at the 95th percentile, 45 % at worst.
 struct Cost {
   float chunk[kNumCfg], chunk_full[kNumCfg], kn[kNumCfg];
   float start, tbs, merge0, merge_rec, merge_split, load;
@@ -73,14 +75,24 @@ constexpr Cost kCostLinear = {{0.139f, 0.308f, 0.366f, 0.426f, 0.507f, 0.612f, 0
                         {0.321f, 0.617f, 0.366f, 0.426f, 0.507f, 0.612f, 0.846f},
                         {1.101f, 0.853f, 0.965f, 1.140f, 1.159f, 1.135f, 1.099f},
                         1.84f, 7.71f, 1.33f, 0.760f, 0.150f, 0.312f};
-constexpr Cost kCostGated = {{0.232f, 0.328f, 0.401f, 0.464f, 1.605f, 0.772f, 1.330f},
-                        {0.564f, 0.645f, 0.401f, 0.464f, 1.605f, 0.772f, 1.330f},
-                        {1.640f, 1.012f, 0.973f, 1.234f, 0.827f, 1.095f, 0.992f},
+constexpr Cost kCostGated = {{0.f, 0.328f, 0.401f, 0.464f, 0.f, 0.772f, 1.330f},  // 0: no tile of the gated MLP
+                        {0.f, 0.645f, 0.401f, 0.464f, 0.f, 0.772f, 1.330f},
+                        {0.f, 1.012f, 0.973f, 1.234f, 0.f, 1.095f, 0.992f},
                         1.67f, 6.88f, 1.25f, 0.666f, 0.147f, 0.176f};
-constexpr Cost kCostNorm = {{0.193f, 0.332f, 0.438f},
-                        {0.421f, 0.332f, 0.438f},
-                        {0.765f, 1.112f, 1.085f},
-                        3.12f, 7.08f, 1.25f, 1.039f, 0.067f, 0.250f};
+// RMSNorm in LDS is fitted to weights that come from HBM, as those of a model's
+// layers do (2410 shapes of 2..315 rows, every tile and split count): 1.0 % on
+// average, 5 % at the 95th percentile, 27 % at worst (5.8, 25 and 65 % with one
+// memory rate for all tiles: it left a quarter of the chip idle where one more
+// split fills it.  8 rows, 4096 x 4096 K x N: 3 splits 12.7 us, 4 12.2; the same
+// weights again 11.2 and 10.7).
+constexpr Cost kCostNorm = {{0.252f, 0.370f, 0.497f},
+                        {0.374f, 0.370f, 0.497f},
+                        {1.073f, 1.002f, 0.956f},
+                        3.624f, 7.08f, 1.135f, 0.499f, 0.156f, 0.329f};
+// its memory rate by layout (N x K, K x N) and tile, and what uneven rounds of
+// the chip add to the memory time (with less than a workgroup per CU, and more)
+constexpr float kNormTbs[2][3] = {{5.609f, 5.669f, 4.600f}, {5.643f, 6.344f, 4.912f}};
+constexpr float kNormFew = 0.458f, kNormUneven = 0.665f;
 
 // Scratch after the tickets: row factors and scaled x of the row pass, then
 // the records of the K splits.
@@ -105,7 +117,8 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
   const bool lds_norm = epi == EPI_RMSNORM && !pass;
   const Cost& c = lds_norm ? kCostNorm : epi == EPI_GATED ? kCostGated : kCostLinear;
   const int nmat = epi == EPI_GATED ? 2 : 1, chunks = (K + KS - 1) / KS;
-  const float mem = 2e-6f * ((float)nmat * K * N + (float)M * K + (float)M * N) / c.tbs;
+  const float mbytes = 2e-6f * ((float)nmat * K * N + (float)M * K + (float)M * N);
+  const int least = lds_norm ? 3 : 5;  // chunks per split (a deep pipeline has to fill)
   float best_t = 3e38f;
   for (int f = 0; f < kNumCfg; f++) {
     const CfgShape& s = kCfg[f];
@@ -122,9 +135,8 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
     const int per_cu = lds_norm && f == C32x128 ? 1 : s.per_cu;
     const float kf = nkl ? 1.f : c.kn[f];
     for (int sp = 1; sp <= kMaxSplits; sp++) {
-      // at least 5 chunks per split (a deep pipeline has to fill), no empty
-      // split, and no more workgroups than a second round of the chip holds
-      if (sp > 1 && (chunks < 5 * sp || tiles * sp > 4 * kCus || tiles > kMaxTickets)) break;
+      // no empty split, and no more workgroups than a second round of the chip holds
+      if (sp > 1 && (chunks < least * sp || tiles * sp > 4 * kCus || tiles > kMaxTickets)) break;
       const int per = (chunks + sp - 1) / sp;
       if ((chunks + per - 1) / per != sp) continue;
       if (split_bytes(f, tiles, sp, lds_norm) > (staged ? most : kSplitBytes)) continue;
@@ -132,6 +144,11 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
       float t = rounds * (per_cu > 1 ? c.chunk_full[f] : c.chunk[f]);
       if (rest) t += rest <= kCus ? c.chunk[f] : c.chunk_full[f];
       t *= per * kf * (1.f + c.load * (wg < kCus ? (float)wg / kCus : 1.f));
+      float mem = mbytes / c.tbs;
+      if (lds_norm) {
+        const float uneven = (float)((wg + kCus - 1) / kCus * kCus) / wg - 1.f;  // the fullest CU over the average
+        mem = mbytes / kNormTbs[nkl ? 0 : 1][f] * (1.f + (wg < kCus ? kNormFew : kNormUneven) * uneven);
+      }
       t = c.start + (t > mem ? t : mem);
       const float rec = s.bm * s.bn * 4.f;  // bytes of a split's record
       if (sp > 1) t += c.merge0 + sp * (c.merge_rec * rec / 65536 + c.merge_split) + 2e-6f * wg * rec / c.tbs;
@@ -144,7 +161,7 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
       }
     }
   }
-  *time = best_t + (pass ? kRowPassUs + 4e-6f * M * K / c.tbs : 0.f);
+  *time = best_t + (pass ? kRowPassUs + 4e-6f * M * K / kRowPassTbs : 0.f);
   return best;
 }
 
