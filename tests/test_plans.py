@@ -80,3 +80,17 @@ def test_few_rows_of_rmsnorm_fill_the_chip():
                 uneven = -(-groups // 256) * 256 / groups
                 worst, total, n = max(worst, uneven), total + uneven, n + 1
     assert worst <= 1.5 and total / n <= 1.2
+
+
+@pytest.mark.parametrize("kind,K,N,kernel", [
+    (_lib.OP_RMSNORM_LINEAR, 2048, 14336, ONE_ROW), (_lib.OP_RMSNORM_LINEAR, 10240, 1024, ONE_ROW),
+    (_lib.OP_RMSNORM_LINEAR, 4096, 4096, ONE_ROW), (_lib.OP_RMSNORM_LINEAR, 4096, 4104, PRODUCT),
+    (_lib.OP_LINEAR, 2048, 8192, ONE_ROW), (_lib.OP_LINEAR, 2048, 8200, PRODUCT),
+    (_lib.OP_LINEAR, 9224, 952, ONE_ROW), (_lib.OP_LINEAR, 14336, 4096, PRODUCT),
+    (_lib.OP_GATED_MLP, 2048, 7168, ONE_ROW), (_lib.OP_GATED_MLP, 2048, 8200, PRODUCT),
+    (_lib.OP_GATED_MLP, 2056, 1024, PRODUCT),
+])
+def test_one_row_of_n_by_k_weights(kind, K, N, kernel):
+    """Both sides of the rule; it never holds for K x N weights or two rows."""
+    assert product_plan(kind, 1, K, N, _lib.W_NK)[0] == kernel
+    assert product_plan(kind, 1, K, N, _lib.W_KN)[0] == product_plan(kind, 2, K, N, _lib.W_NK)[0] == PRODUCT

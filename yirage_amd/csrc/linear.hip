@@ -9,7 +9,7 @@
 //  * K slices of a tile meet through fp32 records: the last workgroup to
 //    arrive (atomic ticket) sums them in slice order.  Deterministic.
 // Its start is short: no LDS stages to fill and, up to K = 2048, no merge.  It
-// is latency-bound there, 4-7 us a launch (rule and figures at one_row()).
+// is latency-bound there, 4-9 us a launch (rule and figures at one_row()).
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -141,21 +141,28 @@ __global__ __launch_bounds__(NK_THREADS) void gemv_nk_kernel(GemvArgs a) {
 
 // ---------------------------------------------------------------- host side
 // One row of x on N x K weights: the one-row kernel while its short start
-// counts, i.e. while one K slice holds K (no merge) and, where there is no
-// norm to wait for, the tiles do not yet fill the chip; past one slice only
-// for small weights.  us, one-row kernel / product kernel:
-//   RMSNorm 2048 x 4096 (K x N) 6.8 / 8.0, 2048 x 8192 9.4 / 11.0,
-//           4096 x 1024 7.1 / 8.6, 4096 x 4096 11.2 / 10.6
-//   linear  2048 x 2048 4.2 / 5.7, 2048 x 8192 7.5 / 7.2, 4096 x 1024 5.9 / 6.6,
-//           4096 x 4096 9.5 / 8.8
-//   gated   2048 x 4096 8.5 / 9.2, 2048 x 8192 12.7 / 11.7, 3072 x 2048 9.6 / 8.9
+// counts, i.e. while one K slice holds K (no merge; without a norm to wait for,
+// as long as the tiles do not pass the chip) and up to 32 MiB of weights; the
+// gated MLP, whose weights are two, only with one slice.  us, one-row kernel /
+// product kernel, weights from HBM (in the cache):
+//   RMSNorm 2048 x 14336 (K x N) 15.6 / 17.2 (13.1 / 12.3), 4096 x 1024 8.9 /
+//           9.3 (7.3 / 8.9), 4096 x 4096 12.7 / 11.9 (8.7 / 10.8), 4096 x 6144
+//           16.2 / 16.1 (14.8 / 14.2)
+//   linear  2048 x 8192 9.5 / 11.0 (4.7 / 6.6), 2048 x 12288 12.6 / 12.9 (8.1 /
+//           9.5), 4096 x 4096 11.1 / 10.6 (6.9 / 7.7), 4096 x 6144 14.9 / 15.5
+//           (13.2 / 11.4), 14336 x 4096 26.5 / 24.4 (22.1 / 19.9)
+//   gated   2048 x 4096 11.1 / 11.8 (6.5 / 9.3), 2048 x 8192 15.9 / 20.5 (13.4 /
+//           12.0), 2048 x 12288 24.2 / 22.3 (19.8 / 16.1), 3072 x 2048 12.1 /
+//           11.5 (8.9 / 7.7)
+// Over 573 shapes the rule is slower than the better of the two by 0.3 %
+// (RMSNorm), 2.2 % (linear) and 3.5 % (gated) on weights from HBM.
 constexpr int kLongK = 1 << 26;  // 32 rows of x reach 4 GiB
 
 static bool one_row(int B, int K, int N, int layout, int epi) {
   if (B != 1 || layout != YR_W_NK) return false;
   if (K >= kLongK) return true;  // the product kernel cuts K in 16 at most, this one in any number of slices
-  if (K <= NK_SLICE) return epi == EPI_RMSNORM || N <= 6144;
-  return epi != EPI_GATED && (long long)K * N <= (epi == EPI_RMSNORM ? 1ll << 23 : 1ll << 22);
+  if (K <= NK_SLICE) return epi == EPI_RMSNORM || N <= 8192;
+  return epi != EPI_GATED && (long long)K * N <= 1ll << 24;
 }
 
 static size_t gemv_workspace(int K, int N, int nmat) {
