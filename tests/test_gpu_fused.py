@@ -113,11 +113,10 @@ def test_gated_mlp_batch128_all_columns():
                                                (33, 1000, 12296, 0, "gated"), (64, 2048, 12296, 1, "rmsnorm"),
                                                (128, 1000, 12296, 0, "rmsnorm")])
 def test_batch128_wide_tiles_and_edges(B, K, N, layout, kind):
-    """Batches of 17..128 rows with N >= 12288: the direct-to-LDS kernel's
-    128-column tiles with two K splits (linear, N x K gated), the last tile 8
-    columns wide (N = 96 * 128 + 8) and a partial 64-row chunk in each split
-    (K = 1000: splits of 512 and 488 rows); RMSNorm runs in the
-    register-staged kernel."""
+    """Batches of 17..128 rows with N >= 12288: the product kernel's tiles of
+    32 and 64 rows and 64 and 128 columns, unsplit, the last one 8 columns wide
+    (N = 96 * 128 + 8), the last 64-k chunk partial (K = 1000), and RMSNorm
+    scaling x in LDS."""
     import yirage_amd.fused as F
 
     print(f"case batch128 {kind} B={B} K={K} N={N} layout={layout}", flush=True)

@@ -1,6 +1,6 @@
-"""GPU parity of the matrix-product kernel (csrc/gemm_kernel.h) at the edges
-of its tiles: rows, columns and K around the tile sizes and the 64-k chunk,
-every epilogue, both weight layouts, one and several K splits.
+"""GPU parity of the matrix-product kernel (csrc/gemm_kernel.h): rows, columns
+and K around the tile sizes and the 64-k chunk, every epilogue, both weight
+layouts, and every tile, whole and with K splits (product_tiles.py).
 
 Reference: float64 products of the same 16-bit inputs, x * gamma rounded to
 the storage type first (the operand the kernels form).  Tolerance: the fp32
@@ -9,6 +9,8 @@ result is rounded once to 16 bits (2^-9 relative for bf16): 1e-2 covers both.
 """
 import pytest
 import torch
+
+from product_tiles import STAGED, TILES
 
 pytestmark = pytest.mark.gpu
 
@@ -35,20 +37,21 @@ def _check(got, ref, what):
 @pytest.mark.parametrize("M,K,N", [
     (1, 8, 8),             # the one-row kernel (N x K)
     (1, 2056, 40),         # its second K slice; the product kernel's for the gated MLP
-    (1, 2048, 6152),       # the other side of its rule for linear and gated
+    (1, 2048, 6152),
+    (1, 2048, 8200),       # the other side of its rule for linear and gated
     (2, 1096, 136),        # the smallest row tile, mostly empty
     (16, 3000, 72),        # many K splits of one column tile
     (17, 8, 8),            # one chunk of 8 k, one column group
     (31, 72, 72),          # a chunk and a piece; a tile and a piece of columns
-    (32, 1000, 520),       # whole rows of the 32-row tiles
-    (33, 1024, 200),       # one row more
+    (32, 1000, 520),       # whole rows of the 32-row tiles, a partial last chunk
+    (33, 1024, 200),       # one row more, whole chunks
     (64, 2056, 136),       # K splits of unequal length
-    (65, 640, 1096),
-    (127, 4096, 72),       # many K splits of one column tile
-    (129, 584, 392),       # RMSNorm by its row pass from here on
-    (250, 1216, 2056),
-    (257, 64, 264),        # one row into the second 256-row tile, a single chunk
-    (600, 1088, 1544),
+    (65, 640, 1096),       # one row more than two 32-row tiles
+    (127, 4096, 72),       # many K splits of two column tiles
+    (129, 584, 392),
+    (250, 1216, 2056),     # the 128-column tiles of 32 and 64 rows
+    (257, 64, 264),        # RMSNorm by its row pass from here on; a single chunk
+    (600, 1088, 1544),     # 32, 64 and, for RMSNorm, 128 rows
 ])
 def test_tile_edges(M, K, N, layout):
     import yirage_amd.fused as F
@@ -71,6 +74,47 @@ def test_tile_edges(M, K, N, layout):
     _check(F.rmsnorm_linear(x, None, w, w_layout=layout), a * rs, "rmsnorm_linear, no gamma")
 
 
+def _run_tile(op, layout, M, K, N, place):
+    """One call of `op` with operands as `place` puts them, twice (the second
+    finds the tickets as the first left them), against float64."""
+    import yirage_amd.fused as F
+
+    print(f"case tile {op} M={M} K={K} N={N} layout={layout}", flush=True)
+    gen = torch.Generator().manual_seed(M + K + N)
+    x, (w, w3), gamma, res = _case(M, K, N, layout, torch.bfloat16 if N % 16 else torch.float16, gen)
+    wd = (w if layout == KN else w.t()).double()
+    if op == "linear":
+        ref = x.double() @ wd + res.double()
+        call = lambda a, b, c: F.linear(a, b, residual=c, w_layout=layout)
+        ops = (x, w, res)
+    elif op == "gated_mlp":
+        a = x.double() @ wd
+        ref = a * torch.sigmoid(a) * (x.double() @ (w3 if layout == KN else w3.t()).double())
+        call = lambda a, b, c: F.gated_mlp(a, b, c, w_layout=layout)
+        ops = (x, w, w3)
+    else:
+        rs = torch.rsqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-6)
+        ref = ((x * gamma).double() @ wd) * rs
+        call = lambda a, b, c: F.rmsnorm_linear(a, c, b, w_layout=layout)
+        ops = (x, w, gamma)
+    ops = [place(t) for t in ops]
+    out = call(*ops)
+    _check(out, ref, op)
+    assert torch.equal(call(*ops), out)
+
+
+@pytest.mark.parametrize("split", [0, 1], ids=["whole", "split"])
+@pytest.mark.parametrize("tile", list(TILES), ids=lambda t: "-".join(map(str, t)))
+def test_every_tile(tile, split):
+    _run_tile(tile[0], tile[1], *TILES[tile][split], lambda t: t)
+
+
+@pytest.mark.parametrize("split", [0, 1], ids=["whole", "split"])
+@pytest.mark.parametrize("tile", list(STAGED), ids=lambda t: "-".join(map(str, t)))
+def test_every_tile_through_registers(tile, split):
+    _run_tile(tile[0], tile[1], *STAGED[tile][split], _odd)
+
+
 def _odd(t):
     """The same values one element off a 16-byte boundary."""
     return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
@@ -78,10 +122,10 @@ def _odd(t):
 
 @pytest.mark.parametrize("layout", [NK, KN])
 @pytest.mark.parametrize("M,K,N", [
-    (1, 4096, 4096),       # product kernel: one row, K splits
+    (1, 4096, 4096),       # N x K: the one-row kernel (not gated); K x N: K splits
     (3, 8, 8),             # a piece of one chunk
     (16, 3000, 72),        # many K splits of one column tile
-    (40, 1096, 200),       # 64-row tile, a partial chunk
+    (40, 1096, 200),       # a partial last chunk
     (130, 584, 392),
     (300, 2056, 264),      # past the rows that scale x in LDS when aligned
 ])

@@ -3,9 +3,11 @@ import ctypes
 
 import pytest
 
+from product_tiles import KN, NK, STAGED, TILES
 from yirage_amd import _lib
 
-ONE_ROW, PRODUCT = 0, 1
+KINDS = {"linear": _lib.OP_LINEAR, "rmsnorm_linear": _lib.OP_RMSNORM_LINEAR, "gated_mlp": _lib.OP_GATED_MLP}
+ONE_ROW, PRODUCT, ATTENTION = 0, 1, 2
 
 
 def product_plan(kind, M, K, N, layout, aligned=True):
@@ -94,3 +96,26 @@ def test_one_row_of_n_by_k_weights(kind, K, N, kernel):
     """Both sides of the rule; it never holds for K x N weights or two rows."""
     assert product_plan(kind, 1, K, N, _lib.W_NK)[0] == kernel
     assert product_plan(kind, 1, K, N, _lib.W_KN)[0] == product_plan(kind, 2, K, N, _lib.W_NK)[0] == PRODUCT
+
+
+def test_every_tile_has_its_shapes():
+    """The shapes of product_tiles.py get the tile they stand for, all tiles are
+    there, and every one of them leaves partial tiles and a partial chunk."""
+    for (op, layout, rows, cols, row_pass), shapes in TILES.items():
+        for split, (M, K, N) in enumerate(shapes):
+            kernel, r, c, s, p, staged = product_plan(KINDS[op], M, K, N, layout)
+            assert (kernel, r, c, s > 1, p, staged) == (PRODUCT, rows, cols, split == 1, row_pass, 0), (op, M, K, N)
+            ncols = cols // 2 if op == "gated_mlp" else cols
+            assert M % rows and N % ncols and K % 64 and (s > 1 or K >= 840)
+    for (op, layout, rows, cols), shapes in STAGED.items():
+        for split, (M, K, N) in enumerate(shapes):
+            kernel, r, c, s, p, staged = product_plan(KINDS[op], M, K, N, layout, aligned=False)
+            assert (kernel, r, c, s > 1, p, staged) == (PRODUCT, rows, cols, split == 1, 0, 1), (op, M, K, N)
+            assert M % rows and N % (cols // 2 if op == "gated_mlp" else cols) and K % 64
+    assert len(STAGED) == 3 * 2 * 2
+    small, large = [(32, 64), (32, 128), (64, 128)], [(128, 128), (128, 192), (128, 256), (256, 256)]
+    for layout in (NK, KN):
+        for r, c in small + large:
+            assert ("linear", layout, r, c, False) in TILES
+            assert ("rmsnorm_linear", layout, r, c, (r, c) in large) in TILES
+            assert (("gated_mlp", layout, r, c, False) in TILES) == ((r, c) not in ((32, 64), (128, 192)))
