@@ -49,8 +49,9 @@ def _check(out, q, k, v, scale):
 @pytest.mark.parametrize("G,M,L,d", [
     (1, 1, 8, 64), (3, 16, 264, 64), (2, 5, 4096, 64),            # 16 rows
     (2, 17, 64, 64), (1, 33, 520, 128), (3, 100, 2040, 128), (4, 64, 4096, 64),  # 32 rows
-    (9, 3601, 72, 128), (260, 65, 8, 128),                        # 64 rows, no split
-    (515, 3, 136, 64), (5, 13001, 72, 64),                        # many groups; 128 rows
+    (9, 3601, 72, 128), (260, 65, 8, 128), (5, 13001, 72, 64),    # 64 rows, no split
+    (5, 13057, 72, 64), (6, 11009, 1544, 64),                     # 128 rows, the last tile 1 row
+    (515, 3, 136, 64),                                            # 16 rows, no split
     (2, 5, 328, 128), (1, 16, 328, 128), (1, 65, 12, 64),         # 12 tokens: packed
 ])
 def test_rows_and_tokens(G, M, L, d, dt):

@@ -119,3 +119,19 @@ def test_every_tile_has_its_shapes():
             assert ("linear", layout, r, c, False) in TILES
             assert ("rmsnorm_linear", layout, r, c, (r, c) in large) in TILES
             assert (("gated_mlp", layout, r, c, False) in TILES) == ((r, c) not in ((32, 64), (128, 192)))
+
+
+@pytest.mark.parametrize("G,M,L,d,rows,split", [
+    (3, 16, 264, 64, 16, True), (515, 3, 136, 64, 16, False), (2, 5, 328, 128, 16, True),
+    (1, 33, 520, 128, 32, True), (4, 64, 4096, 64, 32, True), (260, 65, 8, 128, 64, False),
+    (9, 3601, 72, 128, 64, False), (5, 13001, 72, 64, 64, False), (5, 13057, 72, 64, 128, False),
+    (6, 11009, 1544, 64, 128, False),
+])
+def test_graph_attention_tiles(G, M, L, d, rows, split):
+    """Rows of a workgroup and whether tokens are split; tests/test_gpu_graph_attn.py
+    runs these shapes."""
+    strides = [M * d, d, 1, d * L, L, 1, L * d, d, 1, M * d, d, 1]
+    p = (ctypes.c_int64 * 18)(G, M, L, d, _lib.DTYPE_F16, 0, *strides)
+    plan = (ctypes.c_int * 6)()
+    assert _lib.lib().yr_hip_fused_plan(_lib.OP_ATTENTION, 18, p, 1, plan) == 0, _lib.last_error()
+    assert plan[0] == ATTENTION and plan[1] == rows and (plan[3] > 1) == split, list(plan)
