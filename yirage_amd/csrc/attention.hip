@@ -421,7 +421,8 @@ __device__ __forceinline__ int pf_swz(int row) { return ((row & 7) << 1) | ((row
 // conflicts of the kernel were K reads)
 __device__ __forceinline__ int pk_swz(int row) { return row & 15; }
 
-// HPW heads per wave, HG head groups (of 4 row waves) per workgroup
+// HPW heads per wave (1 is launched: 2 spill registers), HG head groups (of 4
+// row waves) per workgroup
 template <int DT, int HPW, int HG>
 __global__ __launch_bounds__(256 * HG) void gqa_prefill_kernel(PrefillArgs a) {
   constexpr int D = 128;
@@ -904,23 +905,19 @@ int yr::prefill_launch(const char* nm, const void* q, const void* k, const void*
   // heads per workgroup: 2 when the group size allows (two groups of 4 row
   // waves sharing each K / V tile), one head per wave
   const int G = hq / hkv;
-#ifndef YR_PF_CFG
-#define YR_PF_CFG 2
-#endif
-  const int hpw = (YR_PF_CFG == 0 || YR_PF_CFG == 3) && G % 2 == 0 ? 2 : 1;
-  const int hgw = (YR_PF_CFG >= 2) && (G / hpw) % 2 == 0 ? 2 : 1;
+  const int hgw = G % 2 == 0 ? 2 : 1;
   a.paired = a.causal;
   a.npair = a.paired ? (a.nblk + 1) / 2 : a.nblk;
-  a.ngrp = hq / (hpw * hgw);
+  a.ngrp = hq / hgw;
   a.nwg = a.npair * a.ngrp * batch;
   dim3 grid(a.nwg);
   const bool bf = dtype == YR_DTYPE_BF16;
-#define YR_PF(H, W)                                                                                        \
-  if (hpw == H && hgw == W) {                                                                              \
-    if (bf) hipLaunchKernelGGL((gqa_prefill_kernel<DT_BF16, H, W>), grid, dim3(256 * W), 0, st, a);         \
-    else hipLaunchKernelGGL((gqa_prefill_kernel<DT_F16, H, W>), grid, dim3(256 * W), 0, st, a);             \
+#define YR_PF(W)                                                                                           \
+  if (hgw == W) {                                                                                          \
+    if (bf) hipLaunchKernelGGL((gqa_prefill_kernel<DT_BF16, 1, W>), grid, dim3(256 * W), 0, st, a);         \
+    else hipLaunchKernelGGL((gqa_prefill_kernel<DT_F16, 1, W>), grid, dim3(256 * W), 0, st, a);             \
   }
-  YR_PF(1, 1) YR_PF(1, 2) YR_PF(2, 1) YR_PF(2, 2)
+  YR_PF(1) YR_PF(2)
 #undef YR_PF
   YR_CHECK_LAUNCH(nm);
   return YR_OK;
