@@ -13,7 +13,7 @@ kernels instead of searching for and compiling a CUDA program:
       mul(silu(matmul(X, W1)), matmul(X, W3))                       -> gated MLP
       matmul(div(exp(matmul(Q, K)), reduction(exp(.), 2)), V)         -> attention
         (also div(matmul(exp(QK), V), reduction(exp(QK), 2)))
-      matmul(X, W) [+ add(., R)] with 2-D X                          -> skinny linear
+      matmul(X, W) [+ add(., R)] with 2-D X                          -> linear
     and the `customized` threadblock graphs of the reference's demos and
     tests for the first three (demo/reference_mugraphs/*.py);
   * every other op runs on a generic HIP kernel of the same semantics
