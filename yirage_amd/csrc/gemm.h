@@ -29,8 +29,7 @@ struct Call {
 size_t workspace(int M, int K, int N, int epi, bool nkl);
 int run(const Call& c, void* ws, hipStream_t st, const char* name);
 // {YR_PLAN_PRODUCT, tile rows, tile columns, K splits, row pass, operands
-// through registers}
-// of the first launch of a call
+// through registers} of the first launch of a call
 void describe(int M, int K, int N, int epi, bool nkl, bool staged, int* plan6);
 
 // One launch of tile `cfg` (kCfg) with a.splits K splits, `staged` with the

@@ -47,7 +47,8 @@ constexpr int kCus = 256;
 // the model below (71 rows, K 2992, N 3728: 14.9 us against 18.7 with the row
 // pass; 174 rows, K 2928, N 14280: 58.4 against 31.9).  The row pass counts
 // with what such a call takes beyond the model's time for its product (741
-// shapes of 65..315 rows, least squares): 6.3 us and its two streams of x.
+// shapes of 65..315 rows, least squares): 6.3 us and its two streams of x at a
+// rate that holds the product model's own error at these sizes.
 constexpr int kNormLdsAlways = 64, kNormLdsMax = 256;
 constexpr float kRowPassUs = 6.3f, kRowPassTbs = 1.1f;
 constexpr int kPanelRows = 8192;   // rows per launch
@@ -167,7 +168,8 @@ static Plan best_plan(int M, int K, int N, int epi, bool nkl, bool pass, float* 
 
 static Plan make_plan(int M, int K, int N, int epi, bool nkl) {
   float t0 = 0.f, t1 = 0.f;
-  if (epi != EPI_RMSNORM || M <= kNormLdsAlways || (size_t)M * K * 2 > kPassBytes) return best_plan(M, K, N, epi, nkl, false, &t0);
+  if (epi != EPI_RMSNORM || M <= kNormLdsAlways || (size_t)M * K * 2 > kPassBytes)
+    return best_plan(M, K, N, epi, nkl, false, &t0);
   const Plan p = best_plan(M, K, N, epi, nkl, true, &t1);
   if (M > kNormLdsMax) return p;
   const Plan q = best_plan(M, K, N, epi, nkl, false, &t0);
@@ -199,7 +201,7 @@ static Plan plan(int M, int K, int N, int epi, bool nkl, bool staged = false) {
   static thread_local Entry kept[kEntries] = {};
   const int how = 1 + epi * 2 + (nkl ? 1 : 0) + (staged ? 8 : 0);
   Entry& e = kept[((uint32_t)M * 31 + (uint32_t)K * 7 + (uint32_t)N / 8 + how) % kEntries];
-  if (e.M != M || e.K != K || e.N != N || e.how != how) 
+  if (e.M != M || e.K != K || e.N != N || e.how != how)
     e = {M, K, N, how, staged ? make_staged_plan(M, K, N, epi, nkl) : make_plan(M, K, N, epi, nkl)};
   return e.p;
 }
