@@ -5,10 +5,10 @@
  * signatures (streams travel as `void*` holding a hipStream_t; NULL is the
  * null stream).  Every entry point returns YR_OK (0) or a negative YR_E* code;
  * yr_hip_last_error() returns the message of the last failure on the calling
- * thread.  Device pointers must be 16-byte aligned (matrix products, paged
- * decode, argmax and graph attention also take any element address, on slower
- * paths).  All compute calls are stream-ordered and never synchronize the
- * device.
+ * thread.  Device pointers must be 16-byte aligned (the matrix products,
+ * paged decode and argmax also take any element address, the first two on
+ * slower paths).  All compute calls are stream-ordered and never synchronize
+ * the device.
  *
  * Each declaration names the reference interface it replaces
  * (paths relative to the YiRage source tree).
